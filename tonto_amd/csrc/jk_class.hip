@@ -17,11 +17,19 @@
 #define TGPU_SCHWARZ_NAME_X(a, b) TGPU_CAT3(tgpu_launch_schwarz_, a, b)
 #define TGPU_WS_NAME_X(a, b, c, d) TGPU_CAT5(tgpu_wave_ws_, a, b, c, d)
 
-int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, int variant, bool mixed,
-                                                         hipStream_t s)
+// Launches the class pair over `parts` (one per bin pair, every one with bra and ket pairs).
+int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, const JKPart *parts, int n_part,
+                                                         int variant, bool mixed, hipStream_t s)
 {
+    if (n_part <= 0 || n_part > TGPU_MAX_PARTS) return TGPU_OK;
 #if !TGPU_HEAVY
     if (variant == 0) {
+        // parts in the LDS-row form, then the others four bra pairs per work-group
+        JKLaunch rows, glob;
+        rows.a = glob.a = a;
+        rows.n_part = glob.n_part = 0;
+        int rows_grid = 0, glob_grid = 0;
+        size_t lds = 0;
         // The LDS-row form for single molecules with long ket segments (>= 4 rounds of 64 by
         // default, so that the four wavefronts of one bra pair have work): as many of the
         // bra pair's K rows as fit the work-group's LDS budget next to the Rys table and
@@ -30,6 +38,7 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, int 
         // columns of the ket shells' two angular momenta only.  Not built for (ff|ss): its FP64 instantiation
         // gives wrong K on every cluster tested while its mixed twin and the global-atomic
         // form are exact (cause not found), so that class pair updates K globally.
+        bool rows_ok = false;
 #if !(TGPU_LP == 3 && TGPU_LQ == 3 && TGPU_LR == 0 && TGPU_LS == 0)
         constexpr int NP = ncart(TGPU_LP), NQ = ncart(TGPU_LQ);
         constexpr int NRT = EriBody<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, double>::NROOT;
@@ -51,8 +60,9 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, int 
         const int fit = a.kcol_map && W > 0 && budget > kStatic ? (int)((budget - kStatic) / row_bytes) : 0;
         const int nkr = fit < NP + NQ ? fit : NP + NQ;
         // (no K digested, as in the UHF ket-side J pass: no rows)
-        if (a.kp != HUGE_VAL && a.n_ket_avg >= a.krow_min_kets && nkr > 0 && 4 * nkr >= NP + NQ) {
-            JKArgs b = a;
+        rows_ok = a.kp != HUGE_VAL && nkr > 0 && 4 * nkr >= NP + NQ;
+        if (rows_ok) {
+            JKArgs &b = rows.a;
             b.krow_rows = nkr;
             // (..|ss) class pairs: density rows in the LDS left after the K rows, when all
             // of both fit
@@ -60,56 +70,91 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, int 
             b.prow_rows = TGPU_LR == 0 && TGPU_LS == 0 && a.prow_enable && nkr == NP + NQ && pfit >= NP + NQ
                               ? NP + NQ
                               : 0;
-            size_t rows = (size_t)(nkr + b.prow_rows) * row_bytes;
+            lds = (size_t)(nkr + b.prow_rows) * row_bytes;
             // the bra pair's two P_max rows, in what is left, unless they lower the number of
             // work-groups a CU holds ((pp|ss) at 4160 functions: 2 -> 1, 99 -> 130 ms; (ds|ps),
             // at one either way: 259 -> 239 ms)
             const size_t pm_bytes = 2 * (size_t)a.n_shell * sizeof(double);
             constexpr size_t kCuLds = 160 * 1024;
-            b.pmrow = a.pmrow && a.n_shell > 0 && budget >= kStatic + rows + pm_bytes &&
-                              kCuLds / (kStatic + rows + pm_bytes) == kCuLds / (kStatic + rows)
+            b.pmrow = a.pmrow && a.n_shell > 0 && budget >= kStatic + lds + pm_bytes &&
+                              kCuLds / (kStatic + lds + pm_bytes) == kCuLds / (kStatic + lds)
                           ? 1
                           : 0;
-            if (b.pmrow) rows += pm_bytes;
-            if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, true><<<a.n_bra, 256, rows, s>>>(b);
-            else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, true><<<a.n_bra, 256, rows, s>>>(b);
-            return 0;
+            if (b.pmrow) lds += pm_bytes;
         }
 #endif
-        const int blocks = (a.n_bra + 3) / 4;
-        if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, false><<<blocks, 256, 0, s>>>(a);
-        else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, false><<<blocks, 256, 0, s>>>(a);
-        return 0;
+        for (int k = 0; k < n_part; ++k) {
+            const bool r = rows_ok && parts[k].n_ket_avg >= a.krow_min_kets;
+            JKLaunch &L = r ? rows : glob;
+            JKPart &p = L.part[L.n_part++];
+            p = parts[k];
+            p.gx = p.gy = 1;
+            p.first = r ? rows_grid : glob_grid;
+            if (r) rows_grid += p.n_bra;
+            else glob_grid += (p.n_bra + 3) / 4;
+        }
+#if !(TGPU_LP == 3 && TGPU_LQ == 3 && TGPU_LR == 0 && TGPU_LS == 0)
+        if (rows_grid > 0) {
+            if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, true><<<rows_grid, 256, lds, s>>>(rows);
+            else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, true><<<rows_grid, 256, lds, s>>>(rows);
+        }
+#endif
+        if (glob_grid > 0) {
+            if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, false><<<glob_grid, 256, 0, s>>>(glob);
+            else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, false><<<glob_grid, 256, 0, s>>>(glob);
+        }
+        return TGPU_OK;
     }
 #endif
     (void)variant;
     using C = WaveCfg<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS>;
-    // work-group (x, y): bra pairs x, x + gx, ...; of each, ket chunks y, y + gy, ... of
-    // a.ket_chunk kets.  gy splits long prefixes when there are few bra pairs, so that the
-    // grid holds about kWaveGrid work-groups; workspace classes stay within their slots.
+    // work-group (x, y) of a part: bra pairs x, x + gx, ...; of each, ket chunks y, y + gy,
+    // ... of ket_chunk kets.  gy splits long prefixes when there are few bra pairs, so that
+    // a part's grid holds about kWaveGrid work-groups; the launches of workspace classes
+    // stay within their slots, shared evenly by the parts.
     constexpr long long kWaveGrid = 65536;
-    if (a.n_bra <= 0) return 0;
-    const int kc = a.ket_chunk > 0 && a.ket_chunk <= 64 ? a.ket_chunk : 64;  // one lane per ket
-    const long long nch = a.n_ket_max > 0 ? (a.n_ket_max + kc - 1) / kc : 1;
-    long long gx = a.n_bra, gy;
-    if (C::GB) {
-        const long long slots = ws_slot_count(a.ws_doubles, C::WS);
-        // the caller sizes the workspace for at least one slot of every class it launches
-        if (slots <= 0 || !a.ws) return TGPU_E_STATE;
-        gx = std::min<long long>(gx, slots);
-        gy = std::min<long long>(nch, std::max<long long>(1, slots / gx));
-    } else {
-        gy = std::min<long long>(nch, std::max<long long>(1, (kWaveGrid + gx - 1) / gx));
-    }
-    gy = std::min<long long>(gy, 65535);
-    JKArgs b = a;
-    b.ket_chunk = kc;
+    JKLaunch L;
+    L.a = a;
+    L.n_part = n_part;
     // FP64 over the kets before the FP32 split of each prefix (all of it in an FP64 build),
     // then FP32 over the rest
-    if (!mixed) b.fp32_thr = 0.0;
-    jk_wave_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, double><<<dim3((unsigned)gx, (unsigned)gy), 64, 0, s>>>(b);
-    if (mixed) jk_wave_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, float><<<dim3((unsigned)gx, (unsigned)gy), 64, 0, s>>>(b);
-    return 0;
+    if (!mixed) L.a.fp32_thr = 0.0;
+    long long slots = 0;
+    if (C::GB) {
+        slots = ws_slot_count(a.ws_doubles, C::WS);
+        // the caller sizes the workspace for at least one slot of every class it launches;
+        // with fewer slots than parts, each part takes all of them in a launch of its own
+        if (slots <= 0 || !a.ws) return TGPU_E_STATE;
+        if (slots < n_part) {
+            for (int k = 0; k < n_part; ++k)
+                if (int rc = TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(a, parts + k, 1, 1, mixed, s))
+                    return rc;
+            return TGPU_OK;
+        }
+        slots /= n_part;
+    }
+    long long grid = 0;
+    for (int k = 0; k < n_part; ++k) {
+        JKPart &p = L.part[k];
+        p = parts[k];
+        if (p.ket_chunk <= 0 || p.ket_chunk > 64) p.ket_chunk = 64;  // one lane per ket
+        const long long nch = p.n_ket_max > 0 ? (p.n_ket_max + p.ket_chunk - 1) / p.ket_chunk : 1;
+        long long gx = p.n_bra, gy;
+        if (C::GB) {
+            gx = std::min<long long>(gx, slots);
+            gy = std::min<long long>(nch, std::max<long long>(1, slots / gx));
+        } else {
+            gy = std::min<long long>(nch, std::max<long long>(1, (kWaveGrid + gx - 1) / gx));
+        }
+        p.gx = (int)gx;
+        p.gy = (int)gy;
+        p.first = (int)grid;
+        grid += gx * gy;
+    }
+    if (grid > 0x3ffffffLL) return TGPU_E_UNSUPPORTED;  // fewer than 2^32 threads
+    jk_wave_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, double><<<(unsigned)grid, 64, 0, s>>>(L);
+    if (mixed) jk_wave_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, float><<<(unsigned)grid, 64, 0, s>>>(L);
+    return TGPU_OK;
 }
 
 size_t TGPU_WS_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)()

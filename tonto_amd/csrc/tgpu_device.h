@@ -373,6 +373,45 @@ struct JKArgs {
     unsigned long long *counters;
 };
 
+// One launch covers every bin pair of a class pair that runs in the same kernel form: work-
+// group g belongs to the last part with first <= g, and a part's fields replace those of
+// JKArgs.  One launch per class pair instead of one per bin pair (up to 16): the parts fill
+// each other's tails, and a small system pays for 21 launches per build instead of 150.
+#define TGPU_MAX_PARTS (TGPU_NBUCKET * TGPU_NBUCKET)
+struct JKPart {
+    int first;                   // first work-group
+    int bra_start, n_bra, bra_bin, ket_bin, same_bin, ket_chunk, n_ket_max, n_ket_avg;
+    int gx, gy;                  // wavefront form: the part's grid
+    long long kblk_off;
+};
+
+struct JKLaunch {
+    JKArgs a;
+    int n_part;
+    JKPart part[TGPU_MAX_PARTS];
+};
+
+// The work-group's part: its fields into a; returns the work-group's index in the part.
+__device__ __forceinline__ int take_part(const JKLaunch &L, JKArgs &a, int &gx, int &gy)
+{
+    const int g = (int)blockIdx.x;
+    int k = 0;
+    while (k + 1 < L.n_part && L.part[k + 1].first <= g) ++k;  // uniform
+    const JKPart &p = L.part[k];
+    a.bra_start = p.bra_start;
+    a.n_bra = p.n_bra;
+    a.bra_bin = p.bra_bin;
+    a.ket_bin = p.ket_bin;
+    a.same_bin = p.same_bin;
+    a.ket_chunk = p.ket_chunk;
+    a.n_ket_max = p.n_ket_max;
+    a.n_ket_avg = p.n_ket_avg;
+    a.kblk_off = p.kblk_off;
+    gx = p.gx;
+    gy = p.gy;
+    return g - p.first;
+}
+
 // Copies of the J/K accumulators: one per XCD (accelerator complex die).  Device-scope
 // atomics from different XCDs on one cache line move the line between the XCDs' L2
 // caches, one memory write per update; with a copy per XCD each copy's lines are updated
@@ -520,8 +559,11 @@ __device__ __forceinline__ void wave_lds_sync()
 // the other rows are updated with global atomics.  Otherwise four bra pairs per
 // work-group, one per wavefront, and every K update is a global atomic.
 template <int LP, int LQ, int LR, int LS, bool MIXED, bool KROWS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_waves(LP, LQ, LR, LS), 8))) void jk_kernel(JKArgs a)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_waves(LP, LQ, LR, LS), 8))) void jk_kernel(JKLaunch L)
 {
+    JKArgs a = L.a;
+    int gx, gy;  // (the wavefront form's)
+    const int wg = take_part(L, a, gx, gy);
     constexpr int NP = ncart(LP), NQ = ncart(LQ), NR = ncart(LR), NS = ncart(LS);
     constexpr int NPQ = NP * NQ, NRS = NR * NS, NI = NPQ * NRS;
     constexpr int NRT = EriBody<LP, LQ, LR, LS, double>::NROOT;
@@ -538,7 +580,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
     // the bra pair is uniform over the wavefront: readfirstlane lets the compiler keep
     // everything derived from it in scalar registers
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int i = KROWS ? (int)blockIdx.x : (int)blockIdx.x * 4 + wave;
+    const int i = KROWS ? wg : wg * 4 + wave;
     BraInfo b;
     if (KROWS) {
         if (i >= a.n_bra) return;  // uniform over the work-group
@@ -1202,7 +1244,7 @@ __device__ __forceinline__ void wave_digest(const JKArgs &a, const BraInfo &b, c
     }
 }
 
-// The wavefront form's work for bra pair bi: the chunks blockIdx.y, blockIdx.y + gridDim.y,
+// The wavefront form's work for bra pair bi: the chunks y, y + gy,
 // ... of a.ket_chunk kets of its Schwarz prefix (only chunks that hold kets are visited).
 // The 64 lanes screen up to 64 kets of a chunk at once; the kets that pass are then taken
 // TEAMS at a time, one per team (their test results fetched from the lanes that computed
@@ -1211,7 +1253,7 @@ __device__ __forceinline__ void wave_digest(const JKArgs &a, const BraInfo &b, c
 // split, the FP32 one (R = float: tables, accumulation and transfers in FP32) those after
 // it, in a launch of its own, so that neither carries the other's registers.
 template <int LP, int LQ, int LR, int LS, typename R>
-__device__ void wave_bra(const JKArgs &a, int bi, WaveLDS<LP, LQ, LR, LS> *Lt, double *gbuf)
+__device__ void wave_bra(const JKArgs &a, int bi, int y, int gy, WaveLDS<LP, LQ, LR, LS> *Lt, double *gbuf)
 {
     using T = WaveTab<LP, LQ, LR, LS>;
     using C = WaveCfg<LP, LQ, LR, LS>;
@@ -1229,8 +1271,8 @@ __device__ void wave_bra(const JKArgs &a, int bi, WaveLDS<LP, LQ, LR, LS> *Lt, d
         else lo = mid + 1;
     }
     const int jbeg = F32 ? lo : 0, jend = F32 ? b.jend : lo;
-    const int step = gridDim.y * a.ket_chunk;
-    if (jbeg + (int)blockIdx.y * a.ket_chunk >= jend) return;  // uniform over the work-group
+    const int step = gy * a.ket_chunk;
+    if (jbeg + y * a.ket_chunk >= jend) return;  // uniform over the work-group
     const int ld = b.ld, fp = b.fp, fq = b.fq;
     const double *__restrict__ P = b.P;
     for (int t = tl; t < NPQ; t += S) L.Ppq[t] = P[(size_t)(fp + t / NQ) * ld + fq + t % NQ];
@@ -1238,7 +1280,7 @@ __device__ void wave_bra(const JKArgs &a, int bi, WaveLDS<LP, LQ, LR, LS> *Lt, d
 #pragma unroll
     for (int m = 0; m < MJ; ++m) Jpq[m] = 0.0;
     unsigned long long nq = 0, npq = 0;
-    for (int jc = jbeg + blockIdx.y * a.ket_chunk; jc < jend; jc += step) {
+    for (int jc = jbeg + y * a.ket_chunk; jc < jend; jc += step) {
         const int jlim = min(jend, jc + a.ket_chunk);
         KetTest tt;
         const bool ok = jc + lane < jlim && test_ket(a, b, jc + lane, tt);
@@ -1328,20 +1370,23 @@ __device__ void wave_bra(const JKArgs &a, int bi, WaveLDS<LP, LQ, LR, LS> *Lt, d
     __syncthreads();  // L is reused by the work-group's next bra pair
 }
 
-// Wavefront form: grid (gx, gy); work-group (x, y) takes bra pairs x, x + gx, ... and, of
-// each, the ket chunks y, y + gy, ...  Workspace classes keep gx * gy <= their slot count and use
-// slot y * gx + x.
+// Wavefront form: a part's grid is (gx, gy); its work-group (x, y), number y * gx + x, takes
+// bra pairs x, x + gx, ... and, of each, the ket chunks y, y + gy, ...  Workspace classes keep
+// the launch's work-groups <= their slot count and use the work-group's number as slot.
 #ifndef TGPU_WAVE_MIN_WAVES
 #define TGPU_WAVE_MIN_WAVES 1
 #endif
 template <int LP, int LQ, int LR, int LS, typename R>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(TGPU_WAVE_MIN_WAVES, 8))) void jk_wave_kernel(JKArgs a)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(TGPU_WAVE_MIN_WAVES, 8))) void jk_wave_kernel(JKLaunch J)
 {
+    JKArgs a = J.a;
+    int gx, gy;
+    const int wg = take_part(J, a, gx, gy), x = wg % gx, y = wg / gx;
     using C = WaveCfg<LP, LQ, LR, LS>;
     __shared__ WaveLDS<LP, LQ, LR, LS> L[C::TEAMS];
     double *gbuf = nullptr;
-    if constexpr (C::GB) gbuf = a.ws + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * C::WS;
-    for (int bi = blockIdx.x; bi < a.n_bra; bi += gridDim.x) wave_bra<LP, LQ, LR, LS, R>(a, bi, L, gbuf);
+    if constexpr (C::GB) gbuf = a.ws + (size_t)blockIdx.x * C::WS;
+    for (int bi = x; bi < a.n_bra; bi += gx) wave_bra<LP, LQ, LR, LS, R>(a, bi, y, gy, L, gbuf);
 }
 
 template <int LP, int LQ>
@@ -1375,7 +1420,8 @@ __global__ __launch_bounds__(64) void schwarz_wave_kernel(DevPairs pr, DevPrims 
 // Launchers defined in the per-class translation units (jk_class.hip).  variant 0: one
 // lane per quartet (light classes only); variant 1: one wavefront per quartet.
 #define TGPU_DECLARE_JK(LP, LQ, LR, LS, H) \
-    int tgpu_launch_jk_##LP##LQ##LR##LS(const JKArgs &a, int variant, bool mixed, hipStream_t s); \
+    int tgpu_launch_jk_##LP##LQ##LR##LS(const JKArgs &a, const JKPart *parts, int n_part, int variant, \
+                                        bool mixed, hipStream_t s); \
     size_t tgpu_wave_ws_##LP##LQ##LR##LS();
 TGPU_FOR_EACH_CLASS(TGPU_DECLARE_JK)
 #undef TGPU_DECLARE_JK

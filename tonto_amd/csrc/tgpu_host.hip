@@ -1185,7 +1185,7 @@ extern "C" int tgpu_schwarz(tgpu_ctx *c, double *max_I)
     return TGPU_OK;
 }
 
-typedef int (*jk_launcher)(const JKArgs &, int, bool, hipStream_t);
+typedef int (*jk_launcher)(const JKArgs &, const JKPart *, int, int, bool, hipStream_t);
 static const jk_launcher kLaunch[NQCLS] = {
 #define TGPU_LAUNCHER(LP, LQ, LR, LS, H) tgpu_launch_jk_##LP##LQ##LR##LS,
     TGPU_FOR_EACH_CLASS(TGPU_LAUNCHER)
@@ -1306,41 +1306,45 @@ static int enqueue_build(tgpu_ctx *c, const BuildBufs &B, const double *P, doubl
         if (nb == 0 || nk == 0) continue;
         if (prof) (void)hipEventRecord(c->cls_ev[2 * k], s);
         a.counter_slot = k;
-        // every unordered pair of bins once: within one class, ket bucket <= bra bucket
-        for (int bx = 0; bx < NBK; ++bx)
-            for (int by = 0; by < (CX == CY ? bx + 1 : NBK); ++by) {
+        // every unordered pair of bins once: within one class, ket bucket <= bra bucket; the
+        // longest primitive loops first, so that the short ones fill the launch's tail
+        JKPart parts[TGPU_MAX_PARTS];
+        int n_part = 0;
+        int lp = 0;
+        while ((lp + 1) * (lp + 2) / 2 <= CY) ++lp;
+        const int nrs = ncart(lp) * ncart(CY - lp * (lp + 1) / 2);
+        for (int bx = NBK - 1; bx >= 0; --bx)
+            for (int by = (CX == CY ? bx : NBK - 1); by >= 0; --by) {
                 const int X = CX * NBK + bx, Y = CY * NBK + by;
-                a.bra_bin = X;
-                a.ket_bin = Y;
-                a.bra_start = c->bin_start[X];
-                a.n_bra = c->bin_start[X + 1] - c->bin_start[X];
-                a.same_bin = X == Y;
-                a.n_ket_max = c->bin_max_seg[Y];
-                {
-                    int lp = 0;
-                    while ((lp + 1) * (lp + 2) / 2 <= CY) ++lp;
-                    const int nrs = ncart(lp) * ncart(CY - lp * (lp + 1) / 2);
-                    a.kblk_off = c->bin_boff[Y] - (long long)c->bin_start[Y] * nrs;
-                }
+                JKPart p{};
+                p.bra_bin = X;
+                p.ket_bin = Y;
+                p.bra_start = c->bin_start[X];
+                p.n_bra = c->bin_start[X + 1] - c->bin_start[X];
+                p.same_bin = X == Y;
+                p.n_ket_max = c->bin_max_seg[Y];
+                p.kblk_off = c->bin_boff[Y] - (long long)c->bin_start[Y] * nrs;
                 // the LDS-row form is for single large molecules (0 keeps batches of many,
                 // mostly small molecules at four bra pairs per work-group)
-                a.n_ket_avg = c->n_mol == 1 ? c->bin_start[Y + 1] - c->bin_start[Y] : 0;
+                p.n_ket_avg = c->n_mol == 1 ? c->bin_start[Y + 1] - c->bin_start[Y] : 0;
                 // wavefront form: one lane screens each ket of a chunk; the class pair's
                 // tuned chunk (tgpu_autotune), else chunks of 64 unless that leaves fewer
                 // than ~128k work-groups, then 32 or 16
-                a.ket_chunk = 64;
+                p.ket_chunk = 64;
                 if (c->chunk[k] > 0)
-                    a.ket_chunk = c->chunk[k];
+                    p.ket_chunk = c->chunk[k];
                 else
-                    while (a.ket_chunk > 16 &&
-                           (long long)a.n_bra * ((a.n_ket_max + a.ket_chunk - 1) / a.ket_chunk) < 131072)
-                        a.ket_chunk /= 2;
-                if (a.n_bra == 0 || c->bin_start[Y + 1] == c->bin_start[Y]) continue;
-                if (kLaunch[k](a, c->variant[k], mixed, s)) {
-                    c->err = "class pair " + std::to_string(k) + ": no wavefront-form workspace";
-                    return TGPU_E_STATE;
-                }
+                    while (p.ket_chunk > 16 &&
+                           (long long)p.n_bra * ((p.n_ket_max + p.ket_chunk - 1) / p.ket_chunk) < 131072)
+                        p.ket_chunk /= 2;
+                if (p.n_bra == 0 || c->bin_start[Y + 1] == c->bin_start[Y]) continue;
+                parts[n_part++] = p;
             }
+        if (const int rc = kLaunch[k](a, parts, n_part, c->variant[k], mixed, s)) {
+            c->err = "class pair " + std::to_string(k) +
+                     (rc == TGPU_E_STATE ? ": no wavefront-form workspace" : ": too many work-groups");
+            return rc;
+        }
         if (prof) {
             (void)hipEventRecord(c->cls_ev[2 * k + 1], s);
             c->cls_launched[k] = 1;
