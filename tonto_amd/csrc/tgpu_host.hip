@@ -481,6 +481,100 @@ static const bool kWaveDefaultSingle[NQCLS] = {
 #undef TGPU_WAVE_DEFAULT
 };
 
+// The class launches of a build are independent (every update is an atomic add), so they run
+// on the build's stream and kSide side streams, forked from it after the density maxima and
+// joined before post-processing.  Three side streams: with the build's own, one per hardware
+// queue of the process (4).  Small systems gain most (their launches fill a few CUs each):
+// water/6-31G(d) 2.81 -> 1.58 ms, (H2O)8/6-31G(d) 10.5 -> 4.5, (H2O)7/aug-cc-pVDZ J 17.9 ->
+// 9.0; (H2O)32/cc-pVTZ mixed 858 -> 817 (the tails).  A set costs ~2 ms to make, so the sets of a device are shared by
+// its contexts: a call holds one while it enqueues (no other thread puts work on it
+// meanwhile, nor takes part in its capture) and gives it back when the build is enqueued;
+// later builds on the set queue behind.  At most kMost sets per device (a call that finds
+// none runs its launches in series), one kept when the device's last context goes.
+struct SideSet {
+    static constexpr int kSide = 3;
+    hipStream_t s[kSide] = {nullptr, nullptr, nullptr};
+    hipEvent_t fork = nullptr, join[kSide] = {nullptr, nullptr, nullptr};
+
+    bool make()
+    {
+        bool ok = hipEventCreateWithFlags(&fork, hipEventDisableTiming) == hipSuccess;
+        for (int q = 0; q < kSide && ok; ++q)
+            ok = hipStreamCreateWithFlags(&s[q], hipStreamNonBlocking) == hipSuccess &&
+                 hipEventCreateWithFlags(&join[q], hipEventDisableTiming) == hipSuccess;
+        return ok;
+    }
+    ~SideSet()
+    {
+        for (int q = 0; q < kSide; ++q) {
+            if (s[q]) (void)hipStreamDestroy(s[q]);
+            if (join[q]) (void)hipEventDestroy(join[q]);
+        }
+        if (fork) (void)hipEventDestroy(fork);
+    }
+};
+
+struct SidePool {
+    static constexpr int kMost = 8;
+    static std::mutex mu;
+    static std::vector<SideSet *> idle[kMaxDevices];
+    static int made[kMaxDevices], n_ctx[kMaxDevices];
+
+    // an idle set, or (create) a new one on the current device; nullptr if there is none
+    static SideSet *get(int device, bool create)
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        if (!idle[device].empty()) {
+            SideSet *p = idle[device].back();
+            idle[device].pop_back();
+            return p;
+        }
+        int now = -1;
+        if (!create || made[device] >= kMost || hipGetDevice(&now) != hipSuccess || now != device) return nullptr;
+        SideSet *p = new SideSet();
+        if (!p->make()) {
+            delete p;
+            return nullptr;
+        }
+        ++made[device];
+        return p;
+    }
+    static void put(int device, SideSet *p)
+    {
+        if (!p) return;
+        std::lock_guard<std::mutex> lock(mu);
+        idle[device].push_back(p);
+    }
+    static void add_ctx(int device)
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        ++n_ctx[device];
+    }
+    static void drop_ctx(int device)
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        if (--n_ctx[device] > 0) return;
+        while (idle[device].size() > 1) {
+            delete idle[device].back();
+            idle[device].pop_back();
+            --made[device];
+        }
+    }
+};
+std::mutex SidePool::mu;
+std::vector<SideSet *> SidePool::idle[kMaxDevices];
+int SidePool::made[kMaxDevices], SidePool::n_ctx[kMaxDevices];
+
+// A set held by one call
+struct SideLease {
+    const int device;
+    SideSet *const set;
+    SideLease(int d, bool create) : device(d), set(SidePool::get(d, create)) {}
+    ~SideLease() { SidePool::put(device, set); }
+    SideLease(const SideLease &) = delete;
+    SideLease &operator=(const SideLease &) = delete;
+};
+
 struct tgpu_ctx {
     std::string err;
     int device = 0;
@@ -539,6 +633,8 @@ struct tgpu_ctx {
     int prow_enable = 1;      // density rows in LDS in the KROWS form (TGPU_PROW=0: off)
     int pmrow_enable = 1;     // P_max rows in LDS in the KROWS form (TGPU_PMROW=0: off)
     hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_in = nullptr, ev_out = nullptr;
+    double cls_prims[NCLS] = {0.0};  // primitive pairs of each pair class (full lists)
+    bool counted = false;  // in the side streams' context count
     bool timed = false;
     bool profiling = false;
     std::vector<hipEvent_t> cls_ev;  // 2 per class pair
@@ -1008,6 +1104,7 @@ extern "C" int tgpu_destroy(tgpu_ctx *c)
     if (c->ev_out) (void)hipEventDestroy(c->ev_out);
     for (auto &e : c->cls_ev) (void)hipEventDestroy(e);
     if (c->gstream) (void)hipStreamDestroy(c->gstream);
+    if (c->counted) SidePool::drop_ctx(c->device);
     delete c;
     return TGPU_OK;
 }
@@ -1179,6 +1276,15 @@ extern "C" int tgpu_schwarz(tgpu_ctx *c, double *max_I)
             c->maxI_mol[m] = std::max(c->maxI_mol[m], c->maxI[s]);
         }
         if ((rc = dupload(c, c->d_maxI_mol, c->maxI_mol))) return rc;
+        std::fill(c->cls_prims, c->cls_prims + NCLS, 0.0);
+        for (int k = 0; k < NBIN; ++k)
+            for (int s = c->bin_start[k]; s < c->bin_start[k + 1]; ++s) c->cls_prims[k / NBK] += c->n_full[s];
+        // a set of side streams for the builds, made here so that no build has to make one
+        if (!c->counted) {
+            SidePool::add_ctx(c->device);
+            c->counted = true;
+        }
+        SidePool::put(c->device, SidePool::get(c->device, true));
         c->have_schwarz = true;
     }
     if (max_I) std::memcpy(max_I, c->maxI_tonto.data(), sizeof(double) * c->n_pairs);
@@ -1225,12 +1331,62 @@ static size_t workspace_need(const tgpu_ctx *c)
     return need;
 }
 
+// The stream of each class pair of a build: 0 the build's own, 1 .. kSide a side stream,
+// -1 not launched.  Largest first, each to the stream with the least estimated work (the
+// class pair's primitive and contracted quartets before screening, weighted by their table
+// and (e0|f0) work).  The class pairs that use the workspace go to one stream, since they
+// share its slots.  order: the launch order.  Serial (every class pair on stream 0) when
+// `fork` is false.
+static void assign_streams(const tgpu_ctx *c, bool fork, int (&on)[NQCLS], std::vector<int> &order)
+{
+    double cost[NQCLS], ws_cost = 0.0, load[SideSet::kSide + 1] = {0.0};
+    order.clear();
+    for (int k = 0; k < NQCLS; ++k) {
+        const int CX = kClassPair[k][0], CY = kClassPair[k][1];
+        const double nb = c->bin_start[CX * NBK + NBK] - c->bin_start[CX * NBK];
+        const double nk = c->bin_start[CY * NBK + NBK] - c->bin_start[CY * NBK];
+        on[k] = -1;
+        cost[k] = 0.0;
+        if (nb == 0 || nk == 0) continue;
+        on[k] = 0;
+        order.push_back(k);
+        int l[2], ne[2], ni[2], L[2];
+        for (int t = 0; t < 2; ++t) {
+            int lp = 0;
+            while ((lp + 1) * (lp + 2) / 2 <= kClassPair[k][t]) ++lp;
+            l[t] = kClassPair[k][t] - lp * (lp + 1) / 2;
+            L[t] = lp + l[t];
+            ni[t] = ncart(lp) * ncart(l[t]);
+            ne[t] = 0;
+            for (int m = lp; m <= L[t]; ++m) ne[t] += ncart(m);
+        }
+        const double nr = (L[0] + L[1]) / 2 + 1;
+        cost[k] = c->cls_prims[CX] * c->cls_prims[CY] *
+                      (40 + 20 * nr + 9 * nr * (L[0] + 1) * (L[1] + 1) + 3 * nr * ne[0] * ne[1]) +
+                  nb * nk * (100 + 12.0 * ni[0] * ni[1]);
+        if (CX == CY) cost[k] *= 0.5;
+        if (kWaveWs[k]()) ws_cost += cost[k];
+    }
+    if (!fork) return;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost[x] > cost[y]; });
+    load[0] = ws_cost;
+    for (int k : order) {
+        if (kWaveWs[k]()) continue;
+        int q = 0;
+        for (int t = 1; t <= SideSet::kSide; ++t)
+            if (load[t] < load[q]) q = t;
+        on[k] = q;
+        load[q] += cost[k];
+    }
+}
+
 // Enqueue one complete build on stream s (no host synchronisation) into the buffers B.
 // UHF passes: P2 is the other spin's density (screening by max(|P|, |P2|)), j_ket_nonsame
-// selects the J of Tonto's ket side only (and no K).  rec_start / rec_end record the
+// selects the J of Tonto's ket side only (and no K).  side: side streams held by the caller
+// (nullptr: every launch on s).  rec_start / rec_end record the
 // context's timing events around the class launches.
 static int enqueue_build(tgpu_ctx *c, const BuildBufs &B, const double *P, double *J, double *K, int flags,
-                         hipStream_t s, bool rec_start, bool rec_end, const double *P2 = nullptr,
+                         hipStream_t s, SideSet *side, bool rec_start, bool rec_end, const double *P2 = nullptr,
                          int j_ket_nonsame = 0)
 {
     const bool mixed = flags & TGPU_JK_MIXED;
@@ -1298,12 +1454,27 @@ static int enqueue_build(tgpu_ctx *c, const BuildBufs &B, const double *P, doubl
     a.kcol_map = c->n_mol == 1 ? c->d_kcol_map.p : nullptr;
     for (int l = 0; l <= TGPU_LMAX + 1; ++l) a.kcol_lofs[l] = c->kcol_lofs[l];
     const bool prof = rec_end && c->profiling;
-    for (int k = 0; k < NQCLS; ++k) {
+    // one stream where each class pair is timed, and where the caller is capturing s
+    bool fork = side && !prof;
+    if (fork && s && s != c->gstream) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) fork = false;
+    }
+    int on[NQCLS];
+    std::vector<int> order;
+    assign_streams(c, fork, on, order);
+    bool used[SideSet::kSide] = {false, false, false};
+    if (fork) (void)hipEventRecord(side->fork, s);
+    if (prof) std::fill(c->cls_launched.begin(), c->cls_launched.end(), 0);
+    int launch_rc = TGPU_OK;
+    for (const int k : order) {
         const int CX = kClassPair[k][0], CY = kClassPair[k][1];
-        if (prof) c->cls_launched[k] = 0;
-        const int nb = c->bin_start[CX * NBK + NBK] - c->bin_start[CX * NBK];
-        const int nk = c->bin_start[CY * NBK + NBK] - c->bin_start[CY * NBK];
-        if (nb == 0 || nk == 0) continue;
+        hipStream_t sk = s;
+        if (on[k] > 0) {
+            sk = side->s[on[k] - 1];
+            if (!used[on[k] - 1]) (void)hipStreamWaitEvent(sk, side->fork, 0);
+            used[on[k] - 1] = true;
+        }
         if (prof) (void)hipEventRecord(c->cls_ev[2 * k], s);
         a.counter_slot = k;
         // every unordered pair of bins once: within one class, ket bucket <= bra bucket; the
@@ -1340,16 +1511,23 @@ static int enqueue_build(tgpu_ctx *c, const BuildBufs &B, const double *P, doubl
                 if (p.n_bra == 0 || c->bin_start[Y + 1] == c->bin_start[Y]) continue;
                 parts[n_part++] = p;
             }
-        if (const int rc = kLaunch[k](a, parts, n_part, c->variant[k], mixed, s)) {
+        launch_rc = kLaunch[k](a, parts, n_part, c->variant[k], mixed, sk);
+        if (launch_rc) {
             c->err = "class pair " + std::to_string(k) +
-                     (rc == TGPU_E_STATE ? ": no wavefront-form workspace" : ": too many work-groups");
-            return rc;
+                     (launch_rc == TGPU_E_STATE ? ": no wavefront-form workspace" : ": too many work-groups");
+            break;
         }
         if (prof) {
             (void)hipEventRecord(c->cls_ev[2 * k + 1], s);
             c->cls_launched[k] = 1;
         }
     }
+    for (int q = 0; q < SideSet::kSide; ++q)
+        if (used[q]) {
+            (void)hipEventRecord(side->join[q], side->s[q]);
+            (void)hipStreamWaitEvent(s, side->join[q], 0);
+        }
+    if (launch_rc) return launch_rc;
     if (rec_end) (void)hipEventRecord(c->ev1, s);
     if (B.acc_copies > 1)
         acc_reduce_kernel<<<grid_for(c->n_elem), 256, 0, s>>>(B.X, B.Y, (size_t)c->n_elem, B.acc_copies);
@@ -1381,7 +1559,8 @@ extern "C" int tgpu_make_r_JK_device(tgpu_ctx *c, const double *P, double *J, do
     }
     const int kflags = flags & (TGPU_JK_MIXED | TGPU_J_ONLY | TGPU_K_ONLY);
     if (!(flags & TGPU_JK_GRAPH)) {
-        if (int rc = enqueue_build(c, ctx_bufs(c), P, J, K, kflags, c->stream, true, true)) return rc;
+        const SideLease side(c->device, true);
+        if (int rc = enqueue_build(c, ctx_bufs(c), P, J, K, kflags, c->stream, side.set, true, true)) return rc;
         c->timed = true;
         HIPCHK(c, hipGetLastError());
         return TGPU_OK;
@@ -1392,8 +1571,9 @@ extern "C" int tgpu_make_r_JK_device(tgpu_ctx *c, const double *P, double *J, do
         c->g_flags != kflags || c->g_variant != var) {
         drop_graph(c);
         hipGraph_t g = nullptr;
+        const SideLease side(c->device, true);
         HIPCHK(c, hipStreamBeginCapture(c->gstream, hipStreamCaptureModeThreadLocal));
-        const int brc = enqueue_build(c, ctx_bufs(c), P, J, K, kflags, c->gstream, false, false);
+        const int brc = enqueue_build(c, ctx_bufs(c), P, J, K, kflags, c->gstream, side.set, false, false);
         HIPCHK(c, hipStreamEndCapture(c->gstream, &g));
         if (brc) {
             (void)hipGraphDestroy(g);
@@ -1490,7 +1670,8 @@ extern "C" int tgpu_make_r_JK_device_noalloc(tgpu_ctx *c, const double *P, doubl
     B.ws_doubles = ws_slot ? (long long)((TGPU_NOALLOC_SCRATCH_BYTES - off) / sizeof(double)) : 0;
     B.acc_copies = 1;
     const int kflags = flags & (TGPU_JK_MIXED | TGPU_J_ONLY | TGPU_K_ONLY);
-    if (int rc = enqueue_build(c, B, P, J, K, kflags, c->stream, true, true)) return rc;
+    const SideLease side(c->device, false);  // (a new set would be an allocation)
+    if (int rc = enqueue_build(c, B, P, J, K, kflags, c->stream, side.set, true, true)) return rc;
     // the context's own counters take this build's, so tgpu_get_stats reports it
     copy_u64_kernel<<<1, 256, 0, c->stream>>>(c->d_counters.p, B.counters, 3 * NQCLS);
     c->timed = true;
@@ -1533,9 +1714,10 @@ extern "C" int tgpu_make_u_JK_device(tgpu_ctx *c, const double *Pa, const double
     if ((rc = dalloc(c, c->d_uJ, nn)) || (rc = dalloc(c, c->d_uK, nn))) return rc;
     // the timing events bracket all three passes; the class counters are the Pa pass's
     const BuildBufs B = ctx_bufs(c);
-    if ((rc = enqueue_build(c, B, Pb, c->d_uJ.p, c->d_uK.p, flags, c->stream, true, false, Pa, 1)) ||
-        (rc = enqueue_build(c, B, Pb, Jb, Kb, flags, c->stream, false, false, Pa, 0)) ||
-        (rc = enqueue_build(c, B, Pa, Ja, Ka, flags, c->stream, false, true, Pb, 0)))
+    const SideLease side(c->device, true);
+    if ((rc = enqueue_build(c, B, Pb, c->d_uJ.p, c->d_uK.p, flags, c->stream, side.set, true, false, Pa, 1)) ||
+        (rc = enqueue_build(c, B, Pb, Jb, Kb, flags, c->stream, side.set, false, false, Pa, 0)) ||
+        (rc = enqueue_build(c, B, Pa, Ja, Ka, flags, c->stream, side.set, false, true, Pb, 0)))
         return rc;
     uhf_combine_kernel<<<grid_for(nn), 256, 0, c->stream>>>(Ja, Jb, c->d_uJ.p, nn);
     c->timed = true;
@@ -1689,9 +1871,9 @@ extern "C" int tgpu_autotune(tgpu_ctx *c, const double *P, int flags, double *ms
         for (int k = 0; k < NQCLS; ++k) c->variant[k] = kHeavy[k] ? 1 : v;
         // one untimed pass so both forms start from warm caches
         if ((rc = enqueue_build(c, ctx_bufs(c), P, c->d_hJ.p, c->d_hK.p, flags & TGPU_JK_MIXED, c->stream,
-                                false, false)) ||
+                                nullptr, false, false)) ||
             (rc = enqueue_build(c, ctx_bufs(c), P, c->d_hJ.p, c->d_hK.p, flags & TGPU_JK_MIXED, c->stream,
-                                true, true)))
+                                nullptr, true, true)))
             return rc;
         c->timed = true;
         HIPCHK(c, hipGetLastError());
@@ -1710,7 +1892,7 @@ extern "C" int tgpu_autotune(tgpu_ctx *c, const double *P, int flags, double *ms
     for (int q = 0; q < 4; ++q) {
         for (int k = 0; k < NQCLS; ++k) c->chunk[k] = kChunks[q];
         if ((rc = enqueue_build(c, ctx_bufs(c), P, c->d_hJ.p, c->d_hK.p, flags & TGPU_JK_MIXED, c->stream,
-                                true, true)))
+                                nullptr, true, true)))
             return rc;
         c->timed = true;
         HIPCHK(c, hipGetLastError());
