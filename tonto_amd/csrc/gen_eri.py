@@ -12,6 +12,9 @@ relation (a, b+1_t) = (a+1_t, b) + (A-B)_t (a, b) first on the ket side and then
 bra side (`shell1quartet.foo:8310-11134`), writing (pq|rs) as double in the order
 [p][q][r][s] with Tonto's Cartesian component order.
 
+A quartet may be shared by a power-of-two number of neighbouring lanes: each takes a part of
+the ket's primitives and the (e0|f0) sums are added over them before the transfer.
+
 R is the arithmetic type of the recurrences, accumulation and transfer (double or
 float); Rys roots and weights and the primitive prefactors are always FP64.
 
@@ -93,7 +96,8 @@ def gen_class(LP, LQ, LR, LS, R):
     em(f"template <> struct EriBody<{LP}, {LQ}, {LR}, {LS}, {R}> {{", 0)
     em("static constexpr int NP = %d, NQ = %d, NR = %d, NS = %d, NROOT = %d;" % (NP, NQ, NR, NS, nroot))
     em("static __device__ __forceinline__ void run(const DevPrims &pm, const PairView &bra, const PairView &ket,")
-    em("                                           double *__restrict__ out, const double *__restrict__ rys_tab)")
+    em("                                           double *__restrict__ out, const double *__restrict__ rys_tab,")
+    em("                                           int iq0 = 0, int iqs = 1)")
     em("{")
     em(f"{R} G[{NE * NF}];", 2)
     em(f"#pragma unroll", 2)
@@ -101,7 +105,8 @@ def gen_class(LP, LQ, LR, LS, R):
     # outer loop over the ket's primitives (per-lane data, read once each), inner loop over
     # the bra's primitives (the same for the whole wavefront when the caller's bra view
     # is uniform: ldc() then makes them scalar loads)
-    em("for (int iq = 0; iq < ket.n; ++iq) {", 2)
+    # iqs lanes may share the quartet: lane iq0 of them takes the ket primitives iq0, iq0 + iqs, ...
+    em("for (int iq = iq0; iq < ket.n; iq += iqs) {", 2)
     em("const int iqq = ket.off + iq;", 3)
     em("const PrimRec *__restrict__ pk = pm.rec + iqq;", 3)
     em("const double zc = pk->zeta, izc = pk->zinv, Kc = pk->K;", 3)
@@ -158,6 +163,7 @@ def gen_class(LP, LQ, LR, LS, R):
     em("}", 4)
     em("}", 3)
     em("}", 2)
+    em(f"lane_sum<{NE * NF}>(G, iqs);", 2)
     # ---- HRR on ket: G[e][f] -> T[e][r][s]
     Eidx = {c: i for i, c in enumerate(E)}
     Fidx = {c: i for i, c in enumerate(F)}

@@ -174,7 +174,8 @@ void TGPU_SCHWARZ_NAME_X(TGPU_LP, TGPU_LQ)(const DevPairs &pr, const DevPrims &p
 #else
     (void)ws;
     (void)ws_doubles;
-    schwarz_kernel<TGPU_LP, TGPU_LQ><<<(n + 63) / 64, 64, 0, s>>>(pr, pm, start, n, maxI, sph);
+    constexpr int kSplit = 16;
+    schwarz_kernel<TGPU_LP, TGPU_LQ, kSplit><<<(n + 64 / kSplit - 1) / (64 / kSplit), 64, 0, s>>>(pr, pm, start, n, maxI, sph);
 #endif
 }
 #endif

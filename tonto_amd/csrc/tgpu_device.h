@@ -45,6 +45,17 @@ __device__ __forceinline__ T ldc(const T *p)
 #endif
 }
 
+// v[k] summed over groups of n neighbouring lanes (n a power of two, uniform; every lane of a
+// group active), into each of them.
+template <int N, typename R>
+__device__ __forceinline__ void lane_sum(R (&v)[N], int n)
+{
+    for (int off = 1; off < n; off <<= 1) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] += __shfl_xor(v[k], off, 64);
+    }
+}
+
 // One shell pair as the integral code sees it: a run of n primitive pairs starting at
 // off in the primitive arrays (DevPrims), and the pair's A and A - B.  A 32-bit offset
 // rather than six pointers keeps the per-lane state small.
@@ -330,6 +341,9 @@ struct JKArgs {
     DevMols ml;
     int bra_start, n_bra, bra_bin, ket_bin, same_bin, counter_slot, ket_chunk, n_ket_max;
     int n_ket_avg;  // ket-bin pairs of a single molecule (0 for batches)
+    // lane form: log2 of the fewest lanes a quartet is given (more when a group of quartets
+    // leaves lanes idle), and of the most (from the ket bucket's primitive counts)
+    int split, split_max;
     double *ws;    // wavefront-form workspace of ws_doubles doubles: a class uses
     long long ws_doubles;  // min(8192, ws_doubles / WaveCfg::WS) slots
     int max_nbf;   // largest molecule (basis functions)
@@ -382,6 +396,7 @@ struct JKPart {
     int first;                   // first work-group
     int bra_start, n_bra, bra_bin, ket_bin, same_bin, ket_chunk, n_ket_max, n_ket_avg;
     int gx, gy;                  // wavefront form: the part's grid
+    int split, split_max;        // lane form: log2 of the fewest and most lanes per quartet
     long long kblk_off;
 };
 
@@ -407,6 +422,8 @@ __device__ __forceinline__ int take_part(const JKLaunch &L, JKArgs &a, int &gx, 
     a.n_ket_max = p.n_ket_max;
     a.n_ket_avg = p.n_ket_avg;
     a.kblk_off = p.kblk_off;
+    a.split = p.split;
+    a.split_max = p.split_max;
     gx = p.gx;
     gy = p.gy;
     return g - p.first;
@@ -659,7 +676,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
     unsigned long long nq = 0, npq = 0, n32 = 0;
     // one contracted quartet (bra pair, ket j of the prefix) that passed the tests
     // bv: the bra pair's view for this quartet's primitive lists
-    auto quartet = [&](const int j, const int flags, const int fr, const int fs, const PairView &bv) {
+    // sub, ls: the lane is number sub of the 1 << ls lanes that share the quartet
+    auto quartet = [&](const int j, const int flags, const int fr, const int fs, const PairView &bv, const int sub,
+                       const int ls) {
         KetTest t;
         t.sk = b.kb + j;
         t.skipJ = flags & 1;
@@ -669,11 +688,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
         const PairView kv = make_view(a.pr, a.pm, t.sk, t.skip_lists);
         double I[NI];
         if (!MIXED || j < jsplit) {
-            EriBody<LP, LQ, LR, LS, double>::run(a.pm, bv, kv, I, rys_lds);
+            EriBody<LP, LQ, LR, LS, double>::run(a.pm, bv, kv, I, rys_lds, sub, 1 << ls);
         } else {
-            EriBody<LP, LQ, LR, LS, float>::run(a.pm, bv, kv, I, rys_lds);
-            ++n32;
+            EriBody<LP, LQ, LR, LS, float>::run(a.pm, bv, kv, I, rys_lds, sub, 1 << ls);
+            if (sub == 0) ++n32;
         }
+        if (sub) return;  // the group's first lane digests
         ++nq;
         npq += (unsigned long long)(bv.n * kv.n);
         const double f = t.f;
@@ -833,14 +853,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
             wave_lds_sync();
         }
         const bool drain = j0 + step >= b.jend;  // nothing left to test
-        if (qn >= 64 || (drain && qn > 0)) {
-            // take the last min(qn, 64) entries; later rounds append behind the rest
-            const int take = qn < 64 ? qn : 64, base = qn - take;
-            const int2 e = lane < take ? q[base + lane] : make_int2(0, 0);
+        // groups of 64 >> split quartets, each on 1 << split lanes; a smaller last group
+        // takes as many lanes per quartet as it leaves idle
+        const int full = 64 >> a.split;
+        while (qn >= full || (drain && qn > 0)) {
+            // take the last min(qn, full) entries; later rounds append behind the rest
+            const int take = qn < full ? qn : full, base = qn - take;
+            int ls = a.split;
+            while (ls < a.split_max && (take << (ls + 1)) <= 64) ++ls;
+            const int u = lane >> ls;
+            const int2 e = u < take ? q[base + u] : make_int2(0, 0);
             qn = base;
             wave_lds_sync();
-            if (lane < take) quartet(e.x >> 5, e.x & 31, hi16(e.y), lo16(e.y),
-                                     make_view(a.pr, a.pm, b.sb, e.x & 4));
+            if (u < take) quartet(e.x >> 5, e.x & 31, hi16(e.y), lo16(e.y),
+                                  make_view(a.pr, a.pm, b.sb, e.x & 4), lane & ((1 << ls) - 1), ls);
         }
         if (drain && qn == 0) break;
     }
@@ -850,7 +876,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
         KetTest t;
         if (j < b.jend && test_ket(a, b, j, t, pmr, nsh))
             quartet(j, (int)t.skipJ | ((int)t.skipK << 1) | ((int)t.skip_lists << 2) | (t.halvings << 3),
-                    t.fr, t.fs, make_view(a.pr, a.pm, b.sb, t.skip_lists));
+                    t.fr, t.fs, make_view(a.pr, a.pm, b.sb, t.skip_lists), 0, 0);
     }
 #endif
     // wavefront reduction of the bra-pair J block
@@ -888,18 +914,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
 }
 
 // Schwarz table: max_I = sqrt(max |(ab|ab)|) with the full primitive lists
-// (molecule.fock.foo:3712-3752).  One thread per shell pair of one class bin.
-template <int LP, int LQ>
+// (molecule.fock.foo:3712-3752).  SPLIT neighbouring lanes per shell pair of one class bin
+// share its primitives: there are few pairs, and the longest loop (4096 primitive quartets
+// of two contracted s shells) is what the launch waits for.
+template <int LP, int LQ, int SPLIT>
 __global__ __launch_bounds__(64) void schwarz_kernel(DevPairs pr, DevPrims pm, int start, int n,
                                                     double *maxI, int sph)
 {
     constexpr int NP = ncart(LP), NQ = ncart(LQ);
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    const int i = (int)(blockIdx.x * 64 + threadIdx.x) / SPLIT, sub = threadIdx.x & (SPLIT - 1);
+    if (i >= n) return;  // uniform over a pair's lanes
     const int s = start + i;
     const PairView v = make_view(pr, pm, s, false);
     double I[NP * NQ * NP * NQ];
-    EriBody<LP, LQ, LP, LQ, double>::run(pm, v, v, I, rys_table_data + rys_table_offset[EriBody<LP, LQ, LP, LQ, double>::NROOT]);
+    EriBody<LP, LQ, LP, LQ, double>::run(pm, v, v, I, rys_table_data + rys_table_offset[EriBody<LP, LQ, LP, LQ, double>::NROOT],
+                                         sub, SPLIT);
+    if (sub) return;
     double m = 0.0;
     if (sph && (LP >= 2 || LQ >= 2)) {
         // spherical basis: the largest diagonal element of the solid-harmonic block

@@ -1072,7 +1072,6 @@ extern "C" int tgpu_create_batch(const tgpu_system *sys, int n_mol, tgpu_ctx **o
     HIPCHK(c, hipEventCreate(&c->ev1));
     HIPCHK(c, hipEventCreateWithFlags(&c->ev_in, hipEventDisableTiming));
     HIPCHK(c, hipEventCreateWithFlags(&c->ev_out, hipEventDisableTiming));
-    HIPCHK(c, hipStreamCreateWithFlags(&c->gstream, hipStreamNonBlocking));
     return TGPU_OK;
 }
 
@@ -1509,6 +1508,15 @@ static int enqueue_build(tgpu_ctx *c, const BuildBufs &B, const double *P, doubl
                            (long long)p.n_bra * ((p.n_ket_max + p.ket_chunk - 1) / p.ket_chunk) < 131072)
                         p.ket_chunk /= 2;
                 if (p.n_bra == 0 || c->bin_start[Y + 1] == c->bin_start[Y]) continue;
+                // lane form: lanes per quartet, at most about the ket bucket's primitive counts
+                // ({1}, {2-4}, {5-12}, {13+}); as many from the start as it takes to have
+                // kSplitWaves wavefronts
+                static const int kSplitMax[NBK] = {0, 2, 3, 4};
+                constexpr long long kSplitWaves = 4096;
+                p.split_max = kSplitMax[by];
+                const long long waves = (long long)p.n_bra * ((p.n_ket_max + 63) / 64);
+                p.split = 0;
+                while (p.split < p.split_max && (waves << (p.split + 1)) <= kSplitWaves) ++p.split;
                 parts[n_part++] = p;
             }
         launch_rc = kLaunch[k](a, parts, n_part, c->variant[k], mixed, sk);
@@ -1565,7 +1573,10 @@ extern "C" int tgpu_make_r_JK_device(tgpu_ctx *c, const double *P, double *J, do
         HIPCHK(c, hipGetLastError());
         return TGPU_OK;
     }
-    // captured build: (re)capture when the pointers, flags or class variants changed
+    // captured build: (re)capture when the pointers, flags or class variants changed.  (The
+    // stream is made here, not with the context: it would hold one of the process's four
+    // hardware queues, which the side streams use.)
+    if (!c->gstream) HIPCHK(c, hipStreamCreateWithFlags(&c->gstream, hipStreamNonBlocking));
     const std::vector<int> var(c->variant, c->variant + NQCLS);
     if (!c->gexec || c->g_key[0] != P || c->g_key[1] != J || c->g_key[2] != K ||
         c->g_flags != kflags || c->g_variant != var) {
