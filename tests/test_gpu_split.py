@@ -8,6 +8,14 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
+
+@pytest.fixture(autouse=True)
+def torch_cuda():
+    import torch  # before the library: torch brings its own HIP runtime
+    if not torch.cuda.is_available():
+        pytest.fail("no HIP device visible: GPU tests must run on an MI355X")
+
+
 CASES = [(1, "STO-3G"), (1, "6-31G(d)"), (1, "cc-pVDZ"), (2, "cc-pVDZ"), (3, "6-311G(d,p)"), (5, "STO-3G")]
 
 

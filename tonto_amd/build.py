@@ -37,7 +37,7 @@ def class_list():
 
 def _deps(extra):
     return [os.path.join(CSRC, f) for f in ("tgpu_device.h", "rys_table.inc")] + \
-        [os.path.join(CSRC, "gen", "classes.inc"), os.path.join(HERE, "..", "include", "tonto_gpu.h")] + extra
+        [os.path.join(CSRC, "gen", "classes.inc"), os.path.join(CSRC, "gen", "pair_form.inc"), os.path.join(HERE, "..", "include", "tonto_gpu.h")] + extra
 
 
 def _stale(obj, deps):

@@ -18,12 +18,15 @@ the ket's primitives and the (e0|f0) sums are added over them before the transfe
 R is the arithmetic type of the recurrences, accumulation and transfer (double or
 float); Rys roots and weights and the primitive prefactors are always FP64.
 
-Every class also gets `WaveTab<LP, LQ, LR, LS>`: index tables driving the
-wavefront-cooperative kernel (one 64-lane wave per quartet; 2-D tables and HRR levels
-staged in LDS).  Classes with more than HEAVY_NI integrals (or (e0|f0) entries) get only
+The wavefront form (64-lane work-groups, a team of lanes per quartet) is built, for s, p and
+d shells, from `PairForm<L1, L2>`, one per shell-pair class: the (e0|f0) row accumulation
+and the transfer relation of a pair as straight-line code.  Classes with f shells get
+`WaveTab<LP, LQ, LR, LS>` instead: index tables for a kernel that stages the 2-D tables and
+the transfer levels in LDS.  Classes with more than HEAVY_NI integrals (or (e0|f0) entries) get only
 that form.
 
-Output: gen/eri_<LP><LQ><LR><LS>.inc per class and gen/classes.inc, next to this file.
+Output: gen/eri_<LP><LQ><LR><LS>.inc per class, gen/pair_form.inc and gen/classes.inc, next
+to this file.
 """
 import os
 import sys
@@ -33,6 +36,7 @@ from tonto_amd.basis import cart_components  # noqa: E402
 
 LMAX = int(os.environ.get("TGPU_GEN_LMAX", "3"))
 HEAVY_NI = 200
+ROWS_LMAX = 2  # wavefront form: rows and columns in registers up to d shells, levels in LDS above
 
 
 def ncart(l):
@@ -293,6 +297,49 @@ def gen_wave(LP, LQ, LR, LS):
     return "\n".join(out)
 
 
+def gen_pair_form(L1, L2):
+    """PairForm<L1, L2>: the shell-pair operations of the wavefront form as straight-line code.
+
+    acc: G[i] += X[cx] Y[cy] Z[cz] over the components (cx, cy, cz) of l = L1 .. L1 + L2 (one
+    row of (e0|f0), the other index fixed); hrr: the transfer relation from those components
+    to the NO functions of the pair.  comp: the components' exponents."""
+    V = comps_range(L1, L1 + L2)
+    NO = ncart(L1) * ncart(L2)
+    em = Emitter()
+    em(f"template <> struct PairForm<{L1}, {L2}> {{", 0)
+    em(f"static constexpr int L = {L1 + L2}, NV = {len(V)}, NO = {NO};")
+    em(f"static constexpr unsigned char comp[{3 * len(V)}] = {{{', '.join(str(x) for c in V for x in c)}}};")
+    em("template <typename R>")
+    em("static __device__ __forceinline__ void acc(const R (&X)[L + 1], const R (&Y)[L + 1], const R (&Z)[L + 1], R (&G)[NV])")
+    em("{")
+    by_xy = {}
+    for i, c in enumerate(V):
+        by_xy.setdefault(c[:2], []).append((i, c[2]))
+    for (x, y), es in by_xy.items():
+        em(f"{{ const R t = X[{x}] * Y[{y}]; " + " ".join(f"G[{i}] += t * Z[{z}];" for i, z in es) + " }", 2)
+    em("}")
+    em("template <typename R>")
+    em("static __device__ __forceinline__ void hrr(const R (&v)[NV], const R ABx, const R ABy, const R ABz, R (&out)[NO])")
+    em("{")
+    idx = {c: i for i, c in enumerate(V)}
+    axn = "xyz"
+
+    def src(a, b):
+        return f"v[{idx[a]}]" if sum(b) == 0 else "t_%d%d%d_%d%d%d" % (a + b)
+    for lev in hrr_plan(L1, L2):
+        for (dst, sp, s0, t) in lev:
+            em(f"const R {src(*dst)} = {src(*sp)} + AB{axn[t]} * {src(*s0)};", 2)
+    if L2 == 0:
+        em("(void)ABx; (void)ABy; (void)ABz;", 2)
+    sm = cart_components(L2)
+    for ia, a in enumerate(cart_components(L1)):
+        for ib, b in enumerate(sm):
+            em(f"out[{ia * len(sm) + ib}] = {src(a, b)};", 2)
+    em("}")
+    em("};", 0)
+    return "\n".join(em.lines)
+
+
 def classes(lmax):
     pcs = [(lp, lq) for lp in range(lmax + 1) for lq in range(lp + 1)]
     out = []
@@ -308,13 +355,17 @@ def main():
     os.makedirs(gdir, exist_ok=True)
     pcs, qcs = classes(LMAX)
     for (LP, LQ, LR, LS) in qcs:
-        parts = ["/* Generated by gen_eri.py -- do not edit. */",
-                 gen_wave(LP, LQ, LR, LS)]
+        parts = ["/* Generated by gen_eri.py -- do not edit. */"]
+        if LP > ROWS_LMAX:
+            parts.append(gen_wave(LP, LQ, LR, LS))
         if not is_heavy(LP, LQ, LR, LS):
             for R in ("double", "float"):
                 parts.append(gen_class(LP, LQ, LR, LS, R))
         with open(os.path.join(gdir, f"eri_{LP}{LQ}{LR}{LS}.inc"), "w") as f:
             f.write("\n\n".join(parts) + "\n")
+    with open(os.path.join(gdir, "pair_form.inc"), "w") as f:
+        f.write("\n\n".join(["/* Generated by gen_eri.py -- do not edit. */"] +
+                             [gen_pair_form(*p) for p in pcs if p[0] <= ROWS_LMAX]) + "\n")
     lines = ["/* Generated by gen_eri.py -- do not edit. */",
              f"#define TGPU_LMAX {LMAX}",
              f"#define TGPU_NPAIRCLASS {len(pcs)}",

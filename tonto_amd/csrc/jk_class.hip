@@ -107,7 +107,16 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, cons
     }
 #endif
     (void)variant;
+#if TGPU_LP <= 2
+    using namespace rows_form;
+    constexpr bool kGB = false;
+    constexpr long long kWS = 0;
+#else
+    using namespace level_form;
     using C = WaveCfg<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS>;
+    constexpr bool kGB = C::GB;  // transfer buffers in the workspace
+    constexpr long long kWS = C::WS;
+#endif
     // work-group (x, y) of a part: bra pairs x, x + gx, ...; of each, ket chunks y, y + gy,
     // ... of ket_chunk kets.  gy splits long prefixes when there are few bra pairs, so that
     // a part's grid holds about kWaveGrid work-groups; the launches of workspace classes
@@ -120,8 +129,8 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, cons
     // then FP32 over the rest
     if (!mixed) L.a.fp32_thr = 0.0;
     long long slots = 0;
-    if (C::GB) {
-        slots = ws_slot_count(a.ws_doubles, C::WS);
+    if (kGB) {
+        slots = ws_slot_count(a.ws_doubles, kWS);
         // the caller sizes the workspace for at least one slot of every class it launches;
         // with fewer slots than parts, each part takes all of them in a launch of its own
         if (slots <= 0 || !a.ws) return TGPU_E_STATE;
@@ -140,7 +149,7 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, cons
         if (p.ket_chunk <= 0 || p.ket_chunk > 64) p.ket_chunk = 64;  // one lane per ket
         const long long nch = p.n_ket_max > 0 ? (p.n_ket_max + p.ket_chunk - 1) / p.ket_chunk : 1;
         long long gx = p.n_bra, gy;
-        if (C::GB) {
+        if (kGB) {
             gx = std::min<long long>(gx, slots);
             gy = std::min<long long>(nch, std::max<long long>(1, slots / gx));
         } else {
@@ -159,14 +168,24 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, cons
 
 size_t TGPU_WS_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)()
 {
-    return WaveCfg<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS>::WS;
+#if TGPU_LP <= 2
+    return 0;
+#else
+    return level_form::WaveCfg<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS>::WS;
+#endif
 }
 
 #if TGPU_LP == TGPU_LR && TGPU_LQ == TGPU_LS
 void TGPU_SCHWARZ_NAME_X(TGPU_LP, TGPU_LQ)(const DevPairs &pr, const DevPrims &pm, int start, int n,
                                           double *maxI, double *ws, long long ws_doubles, int sph, hipStream_t s)
 {
-#if TGPU_HEAVY
+#if TGPU_HEAVY && TGPU_LP <= 2
+    (void)ws;
+    (void)ws_doubles;
+    constexpr int T = rows_form::WaveCfg<TGPU_LP, TGPU_LQ, TGPU_LP, TGPU_LQ>::TEAMS;
+    rows_form::schwarz_wave_kernel<TGPU_LP, TGPU_LQ><<<(n + T - 1) / T, 64, 0, s>>>(pr, pm, start, n, maxI, sph);
+#elif TGPU_HEAVY
+    using namespace level_form;
     using C = WaveCfg<TGPU_LP, TGPU_LQ, TGPU_LP, TGPU_LQ>;
     const long long slots = ws_slot_count(ws_doubles, C::WS);
     const int grid = C::GB ? (int)(n < slots ? n : slots) : n;

@@ -945,18 +945,524 @@ __global__ __launch_bounds__(64) void schwarz_kernel(DevPairs pr, DevPrims pm, i
 }
 
 
-// ----------------------------------------------------------------------------------
-// Heavy classes: one 64-lane wavefront (= one work-group) per quartet.
-// Per primitive quartet, lanes (axis, root) build the 2-D Rys tables into LDS and every
-// lane accumulates its slice of the (e0|f0) entries in registers; the ket-side and then
-// the bra-side transfer relation run level by level in LDS with lanes over entries;
-// the digestion gives each J/K target element to one lane (one atomic per element).
-// ----------------------------------------------------------------------------------
+// index of the (k+1)-th set bit of m (64 if there is none)
+__device__ __forceinline__ int nth_set_bit(unsigned long long m, int k)
+{
+    for (int i = 0; i < k && m; ++i) m &= m - 1;
+    return m ? __builtin_ctzll(m) : 64;
+}
+
 // slots of a workspace class: one per resident work-group of its persistent grid
 __host__ __device__ constexpr long long ws_slot_count(long long ws_doubles, long long per_slot)
 {
     return per_slot <= 0 ? 0 : (ws_doubles / per_slot < 8192 ? ws_doubles / per_slot : 8192);
 }
+
+namespace rows_form {
+// ----------------------------------------------------------------------------------
+// Wavefront form of the classes of s, p and d shells: one 64-lane wavefront (= one work-group)
+// on 1, 2 or 4 quartets, in registers.
+//
+// A quartet's team of S lanes goes through three layouts, so that all but the 2-D tables,
+// the half-transferred block and the K partial sums stays in registers:
+//   tables   per primitive quartet, lanes (axis, root) build the 2-D Rys tables into LDS;
+//   rows     lane e owns row e of (e0|f0): it reads 3 (LRS + 1) table entries per root (not 3
+//            per (e0|f0) element), accumulates the row in registers and transfers the ket
+//            there; (e0|rs) goes to LDS, and its product with the ket's density joins the
+//            lane's W(e), from which the bra pair's J block is transferred once, after all
+//            kets (the transfer is linear and A - B is the bra pair's);
+//   columns  lane c = (r, s) reads column c of (e0|rs), transfers the bra in registers and
+//            digests its NPQ integrals there: ket-side J by one atomic, K as partial sums
+//            over q or p, through LDS, added over s or r by one lane per K element.
+// LDS holds NE NRS values a quartet instead of two buffers of up to 1.5 NPQ NRS, so that 2 to
+// 3 wavefronts fit a SIMD.  The classes with f shells keep the level form below: their rows
+// and columns (25 to 100 values a lane) do not fit the registers.
+// ----------------------------------------------------------------------------------
+template <int L1, int L2> struct PairForm;
+#include "gen/pair_form.inc"
+
+template <int LP, int LQ, int LR, int LS>
+struct WaveCfg {
+    using B = PairForm<LP, LQ>;
+    using K = PairForm<LR, LS>;
+    static constexpr int NP = ncart(LP), NQ = ncart(LQ), NR = ncart(LR), NS = ncart(LS);
+    static constexpr int NE = B::NV, NF = K::NV, NPQ = B::NO, NRS = K::NO;
+    static constexpr int NROOT = (B::L + K::L) / 2 + 1, W1 = B::L + 1, W2 = K::L + 1;
+    static constexpr int NGT = 3 * NROOT * W1 * W2;  // 2-D tables of a primitive quartet
+    // lanes of a team: they cover the 3n (axis, root) tasks and, up to 64, the rows and the
+    // columns
+    static constexpr int S = NE <= 16 && NRS <= 16 && 3 * NROOT <= 16 ? 16 : NE <= 32 && NRS <= 32 ? 32 : 64;
+    static constexpr int TEAMS = 64 / S;
+    static constexpr int EP = (NE + S - 1) / S, CP = (NRS + S - 1) / S;  // passes over rows, columns
+    // primitive quartets per table phase (at most two)
+    static constexpr int PB = 2 * 3 * NROOT <= S ? 2 : 1;
+    // (e0|rs): rows of LD values, LD odd so that the lanes' rows start in different banks
+    static constexpr int LD = NRS | 1;
+    static constexpr int NK = 2 * (NP + NQ) * NRS;  // K partial sums
+};
+
+// One team's LDS: tables and (e0|rs) in the quartet's arithmetic type R; the K partial sums
+// take their place once every lane has read its column (a class with more columns than
+// lanes keeps them apart); the density blocks of the quartet.
+template <int LP, int LQ, int LR, int LS, typename R>
+struct WaveBuf {
+    using C = WaveCfg<LP, LQ, LR, LS>;
+    R g[C::PB * C::NGT];
+    R h[C::NE * C::LD];
+};
+template <int LP, int LQ, int LR, int LS>
+struct WaveLDS {
+    using C = WaveCfg<LP, LQ, LR, LS>;
+    union {
+        WaveBuf<LP, LQ, LR, LS, double> d;
+        WaveBuf<LP, LQ, LR, LS, float> f;
+        double k[C::CP == 1 ? C::NK : 1];
+    } u;
+    double kfar[C::CP == 1 ? 1 : C::NK];
+    double Prs[C::NRS];
+    double Psq[C::NS * C::NQ], Prq[C::NR * C::NQ], Psp[C::NS * C::NP], Prp[C::NR * C::NP];
+};
+
+template <int LP, int LQ, int LR, int LS, typename R>
+__device__ __forceinline__ WaveBuf<LP, LQ, LR, LS, R> &wave_buf(WaveLDS<LP, LQ, LR, LS> &L)
+{
+    if constexpr (sizeof(R) == sizeof(double)) return L.u.d;
+    else return L.u.f;
+}
+
+// Offsets of the lane's rows e in one axis's table of one root: W2 times the exponents of
+// component e, x | y << 8 | z << 16.
+template <int LP, int LQ, int LR, int LS>
+__device__ __forceinline__ void row_offsets(int tl, int (&rows)[WaveCfg<LP, LQ, LR, LS>::EP])
+{
+    using C = WaveCfg<LP, LQ, LR, LS>;
+#pragma unroll
+    for (int m = 0; m < C::EP; ++m) {
+        const int e = tl + C::S * m < C::NE ? tl + C::S * m : 0;
+        const unsigned char *cp = C::B::comp + 3 * e;
+        rows[m] = (cp[0] | cp[1] << 8 | cp[2] << 16) * C::W2;
+    }
+}
+
+// (e0|rs) of one contracted quartet per team, into B.h.  R is the type of the 2-D tables,
+// the accumulation and the transfer; roots, weights and the recurrence coefficients are
+// computed in FP64.  All lanes of the wavefront call it together; tl is the lane's index in
+// its team, B the team's buffers.  A team without a quartet (not live) follows along; np is
+// the quartet's primitive-quartet count (0 also where every primitive pair was dropped: the
+// integrals are then zero), npmax, the largest over the teams, is uniform.  row(pass, out): called
+// by the lane of each row with the row's NRS values.
+// rows: where the lane's rows lie in the tables (row_offsets).
+template <int LP, int LQ, int LR, int LS, typename R, typename Row>
+__device__ __forceinline__ void wave_rows(const DevPrims &pm, const PairView &bra, const PairView &ket,
+                                          const int (&rows)[WaveCfg<LP, LQ, LR, LS>::EP],
+                                          WaveBuf<LP, LQ, LR, LS, R> &B, int tl, bool live, int np, int npmax, Row &&row)
+{
+    using C = WaveCfg<LP, LQ, LR, LS>;
+    using KF = typename C::K;
+    constexpr int N = C::NROOT, W1 = C::W1, W2 = C::W2, TW = W1 * W2, S = C::S, PB = C::PB;
+    // the lane's table task
+    const int tb = tl / (3 * N), task = tl - tb * (3 * N), ax = task / N, rr = task - ax * N;
+#pragma unroll 1
+    for (int pass = 0; pass < C::EP; ++pass) {
+        const int e = tl + S * pass;
+        const bool own = e < C::NE;
+        int ro = rows[0];
+#pragma unroll
+        for (int k = 1; k < C::EP; ++k) ro = pass == k ? rows[k] : ro;
+        const int xo = ro & 255, yo = ((ro >> 8) & 255) + N * TW, zo = (ro >> 16) + 2 * N * TW;
+        R G[C::NF];
+#pragma unroll
+        for (int k = 0; k < C::NF; ++k) G[k] = (R)0;
+        int iq = 0, ip = tb;  // the task's primitive pair of ket and bra
+#pragma unroll 1
+        for (int i0 = 0; i0 < npmax; i0 += PB) {
+            if (tl < 3 * N * PB && i0 + tb < np) {
+                while (ip >= bra.n) {
+                    ip -= bra.n;
+                    ++iq;
+                }
+                const PrimRec pb = ldc(pm.rec + bra.off + ip);
+                const PrimRec pk = ldc(pm.rec + ket.off + iq);
+                ip += PB;
+                const double za = pb.zeta, zc = pk.zeta;
+                const double izs = 1.0 / (za + zc), rz0 = zc * izs, re0 = za * izs, rho = za * rz0;
+                const double QP[3] = {pk.Px - pb.Px, pk.Py - pb.Py, pk.Pz - pb.Pz};
+                const double X = rho * (QP[0] * QP[0] + QP[1] * QP[1] + QP[2] * QP[2]);
+                double ur, wr;
+                rys_root_one<N>(X, rr, ur, wr);
+                const double PA = ax == 0 ? pb.Px - bra.Ax : ax == 1 ? pb.Py - bra.Ay : pb.Pz - bra.Az;
+                const double QC = ax == 0 ? pk.Px - ket.Ax : ax == 1 ? pk.Py - ket.Ay : pk.Pz - ket.Az;
+                const double qp = ax == 0 ? QP[0] : ax == 1 ? QP[1] : QP[2];
+                const double rz = ur * rz0, re = ur * re0;
+                const R b10 = (R)((1.0 - rz) * 0.5 * pb.zinv), b01 = (R)((1.0 - re) * 0.5 * pk.zinv),
+                        b00 = (R)(ur * 0.5 * izs);
+                const R c00 = (R)(PA + rz * qp), d00 = (R)(QC - re * qp);
+                // the 2-D table I(e, f) column by column (two columns live), each column
+                // stored to LDS as soon as it is complete
+                R *gt = B.g + tb * C::NGT + (ax * N + rr) * TW;
+                R cl[W1], cc[W1];
+                cc[0] = ax == 2 ? (R)(wr * (TWOPI5ON2 * pb.K * pk.K * sqrt(rho))) : (R)1;
+#pragma unroll
+                for (int m = 0; m + 1 < W1; ++m) cc[m + 1] = c00 * cc[m] + (m ? (R)m * b10 * cc[m - 1] : (R)0);
+#pragma unroll
+                for (int m = 0; m < W1; ++m) gt[m * W2] = cc[m];
+#pragma unroll
+                for (int f = 0; f + 1 < W2; ++f) {
+                    R cn[W1];
+#pragma unroll
+                    for (int m = 0; m < W1; ++m)
+                        cn[m] = d00 * cc[m] + (f ? (R)f * b01 * cl[m] : (R)0) + (m ? (R)m * b00 * cc[m - 1] : (R)0);
+#pragma unroll
+                    for (int m = 0; m < W1; ++m) {
+                        gt[m * W2 + f + 1] = cn[m];
+                        cl[m] = cc[m];
+                        cc[m] = cn[m];
+                    }
+                }
+            }
+            wave_lds_sync();
+#pragma unroll
+            for (int b = 0; b < PB; ++b) {
+                if (own && i0 + b < np) {
+#pragma unroll(C::NF <= 16 ? N : 1)
+                    for (int r = 0; r < N; ++r) {
+                        const R *gr = B.g + b * C::NGT + r * TW;
+                        R X[W2], Y[W2], Z[W2];
+#pragma unroll
+                        for (int f = 0; f < W2; ++f) {
+                            X[f] = gr[xo + f];
+                            Y[f] = gr[yo + f];
+                            Z[f] = gr[zo + f];
+                        }
+                        KF::acc(X, Y, Z, G);
+                    }
+                }
+            }
+            wave_lds_sync();
+        }
+        if (own && live) {
+            R out[C::NRS];
+            KF::hrr(G, (R)ket.ABx, (R)ket.ABy, (R)ket.ABz, out);
+            R *hr = B.h + e * C::LD;
+#pragma unroll
+            for (int c = 0; c < C::NRS; ++c) hr[c] = out[c];
+            row(pass, out);
+        }
+    }
+    wave_lds_sync();
+}
+
+// Column c of (e0|rs) transferred to the bra's functions
+template <int LP, int LQ, int LR, int LS, typename R>
+__device__ __forceinline__ void wave_column(const PairView &bra, const WaveBuf<LP, LQ, LR, LS, R> &B, int c,
+                                            R (&I)[WaveCfg<LP, LQ, LR, LS>::NPQ])
+{
+    using C = WaveCfg<LP, LQ, LR, LS>;
+    R v[C::NE];
+#pragma unroll
+    for (int e = 0; e < C::NE; ++e) v[e] = B.h[e * C::LD + c];
+    C::B::hrr(v, (R)bra.ABx, (R)bra.ABy, (R)bra.ABz, I);
+}
+
+
+// The wavefront form's work for bra pair bi: the chunks y, y + gy,
+// ... of a.ket_chunk kets of its Schwarz prefix (only chunks that hold kets are visited).
+// The 64 lanes screen up to 64 kets of a chunk at once; the kets that pass are then taken
+// TEAMS at a time, one per team (their test results fetched from the lanes that computed
+// them).  The prefix is split where max_I(ab) max_I(cd) falls below a.fp32_thr (0 in an
+// FP64 build: no split): the FP64 instantiation (R = double) takes the kets before the
+// split, the FP32 one (R = float: tables, accumulation and transfers in FP32) those after
+// it, in a launch of its own, so that neither carries the other's registers.
+template <int LP, int LQ, int LR, int LS, typename R>
+__device__ void wave_bra(const JKArgs &a, int bi, int y, int gy, WaveLDS<LP, LQ, LR, LS> *Lt, double *Lbra)
+{
+    using C = WaveCfg<LP, LQ, LR, LS>;
+    constexpr bool F32 = sizeof(R) == sizeof(float);
+    constexpr int NP = C::NP, NQ = C::NQ, NR = C::NR, NS = C::NS, S = C::S, NT = C::TEAMS;
+    constexpr int NPQ = C::NPQ, NRS = C::NRS, NE = C::NE;
+    const int lane = threadIdx.x, team = lane / S, tl = lane - team * S;
+    WaveLDS<LP, LQ, LR, LS> &L = Lt[team];
+    WaveBuf<LP, LQ, LR, LS, R> &B = wave_buf<LP, LQ, LR, LS, R>(L);
+    double *const kt = C::CP == 1 ? L.u.k : L.kfar;
+    BraInfo b;
+    load_bra(a, bi, b);
+    int lo = 0, hi = b.jend;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (b.mIb * ldc(b.maxI + mid) < a.fp32_thr) hi = mid;
+        else lo = mid + 1;
+    }
+    const int jbeg = F32 ? lo : 0, jend = F32 ? b.jend : lo;
+    const int step = gy * a.ket_chunk;
+    if (jbeg + y * a.ket_chunk >= jend) return;  // uniform over the work-group
+    const int ld = b.ld, fp = b.fp, fq = b.fq;
+    const double *__restrict__ P = b.P;
+    // the bra pair's density block, shared by the teams
+    for (int t = lane; t < NPQ; t += 64) Lbra[t] = P[(size_t)(fp + t / NQ) * ld + fq + t % NQ];
+    int rows[C::EP];
+    row_offsets<LP, LQ, LR, LS>(tl, rows);
+    double W[C::EP];
+#pragma unroll
+    for (int m = 0; m < C::EP; ++m) W[m] = 0.0;
+    unsigned long long nq = 0, npq = 0;
+    for (int jc = jbeg + y * a.ket_chunk; jc < jend; jc += step) {
+        const int jlim = min(jend, jc + a.ket_chunk);
+        KetTest tt;
+        const bool ok = jc + lane < jlim && test_ket(a, b, jc + lane, tt);
+        const int flags_l = ok ? ((int)tt.skipJ | ((int)tt.skipK << 1) | ((int)tt.skip_lists << 2) |
+                                  (tt.halvings << 3))
+                               : 0;
+        const int frs_l = ok ? pack16(tt.fr, tt.fs) : 0;
+        unsigned long long pass = __ballot(ok);
+        while (pass) {  // uniform over the work-group
+            // this round: the team-th remaining ket for each team
+            const int l = nth_set_bit(pass, team);
+            const bool live = l < 64;
+#pragma unroll
+            for (int k = 0; k < NT; ++k) pass &= pass - 1;
+            const int src_lane = live ? l : 0;
+            const int flags = __shfl(flags_l, src_lane, 64), frs = __shfl(frs_l, src_lane, 64);
+            const int sk = b.kb + jc + src_lane;
+            const bool do_J = live && !(flags & 1), do_K = live && !(flags & 2), skip_lists = flags & 4;
+            const double f = (flags >> 3) == 0 ? 1.0 : (flags >> 3) == 1 ? 0.5 : (flags >> 3) == 2 ? 0.25 : 0.125;
+            const PairView bv = make_view(a.pr, a.pm, b.sb, skip_lists);
+            const PairView kv = make_view(a.pr, a.pm, sk, skip_lists);
+            const int fr = hi16(frs), fs = lo16(frs);
+            // J sides as in the lane form (both, or the UHF pass's Tonto ket side only)
+            bool j_ket = do_J, j_bra = do_J;
+            if (a.j_ket_nonsame) {
+                const int tk = ldc(a.pr.rec0 + sk).x;
+                j_ket = do_J && b.tb > tk;
+                j_bra = do_J && b.tb < tk;
+            }
+            const long long kblk = a.kblk_off + (long long)sk * NRS;
+            // stage the ket-dependent density blocks (P symmetric: the K-side blocks come from
+            // the bra pair's rows)
+            if (live) {
+                if constexpr (NRS <= S && NS * NQ <= S && NR * NQ <= S && NS * NP <= S && NR * NP <= S) {
+                    // one pass of the team's lanes: the five loads are in flight together
+                    const int u = tl;
+                    const double v0 = u < NRS ? a.PP[kblk + u] : 0.0;
+                    const double v1 = u < NS * NQ ? P[(size_t)(fq + u % NQ) * ld + fs + u / NQ] : 0.0;
+                    const double v2 = u < NR * NQ ? P[(size_t)(fq + u % NQ) * ld + fr + u / NQ] : 0.0;
+                    const double v3 = u < NS * NP ? P[(size_t)(fp + u % NP) * ld + fs + u / NP] : 0.0;
+                    const double v4 = u < NR * NP ? P[(size_t)(fp + u % NP) * ld + fr + u / NP] : 0.0;
+                    if (u < NRS) L.Prs[u] = v0;
+                    if (u < NS * NQ) L.Psq[u] = v1;
+                    if (u < NR * NQ) L.Prq[u] = v2;
+                    if (u < NS * NP) L.Psp[u] = v3;
+                    if (u < NR * NP) L.Prp[u] = v4;
+                } else {
+                    for (int u = tl; u < NRS; u += S) L.Prs[u] = a.PP[kblk + u];
+                    for (int u = tl; u < NS * NQ; u += S) L.Psq[u] = P[(size_t)(fq + u % NQ) * ld + fs + u / NQ];
+                    for (int u = tl; u < NR * NQ; u += S) L.Prq[u] = P[(size_t)(fq + u % NQ) * ld + fr + u / NQ];
+                    for (int u = tl; u < NS * NP; u += S) L.Psp[u] = P[(size_t)(fp + u % NP) * ld + fs + u / NP];
+                    for (int u = tl; u < NR * NP; u += S) L.Prp[u] = P[(size_t)(fp + u % NP) * ld + fr + u / NP];
+                }
+            }
+            // primitive quartets of the longest quartet this round (uniform loop bound)
+            const int np = live ? bv.n * kv.n : 0;
+            int npmax = np;
+#pragma unroll
+            for (int off = 32; off >= S; off >>= 1) npmax = max(npmax, __shfl_xor(npmax, off, 64));
+            wave_lds_sync();
+            wave_rows<LP, LQ, LR, LS, R>(a.pm, bv, kv, rows, B, tl, live, np, npmax, [&](int m, const R(&out)[NRS]) {
+                if (j_bra) {
+                    double acc = 0.0;
+#pragma unroll
+                    for (int c = 0; c < NRS; ++c) acc += (double)out[c] * L.Prs[c];
+#pragma unroll
+                    for (int k = 0; k < C::EP; ++k)
+                        if (k == m) W[k] += f * acc;
+                }
+            });
+#pragma unroll 1
+            for (int cpass = 0; cpass < C::CP; ++cpass) {
+                const int c = tl + S * cpass;
+                const bool own = live && c < NRS;
+                R I[NPQ];
+                if (own) wave_column<LP, LQ, LR, LS, R>(bv, B, c, I);
+                // every column is read before the K sums replace (e0|rs)
+                wave_lds_sync();
+                if (own && j_ket) {
+                    double acc = 0.0;
+#pragma unroll
+                    for (int pq = 0; pq < NPQ; ++pq) acc += (double)I[pq] * Lbra[pq];
+                    unsafeAtomicAdd(&a.XP[kblk + c], f * acc);
+                }
+                if (own && do_K) {
+                    // partial sums of K(p,r) += I P(s,q), K(p,s) += I P(r,q) over q, and of
+                    // K(q,r) += I P(s,p), K(q,s) += I P(r,p) over p
+                    const int r = c / NS, s = c - r * NS;
+                    double T3[NQ], T4[NQ];
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) T3[q] = T4[q] = 0.0;
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) {
+                        const double ps = L.Psp[s * NP + p], pr = L.Prp[r * NP + p];
+                        double T1 = 0.0, T2 = 0.0;
+#pragma unroll
+                        for (int q = 0; q < NQ; ++q) {
+                            const double v = (double)I[p * NQ + q];
+                            T1 += v * L.Psq[s * NQ + q];
+                            T2 += v * L.Prq[r * NQ + q];
+                            T3[q] += v * ps;
+                            T4[q] += v * pr;
+                        }
+                        kt[(2 * p) * NRS + c] = T1;
+                        kt[(2 * p + 1) * NRS + c] = T2;
+                    }
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) {
+                        kt[(2 * (NP + q)) * NRS + c] = T3[q];
+                        kt[(2 * (NP + q) + 1) * NRS + c] = T4[q];
+                    }
+                }
+            }
+            wave_lds_sync();
+            if (do_K) {
+                // one lane per K element: row x of the bra pair, function y of the ket pair
+                constexpr int NY = NR + NS, NX = NP + NQ;
+                for (int u = tl; u < NX * NY; u += S) {
+                    const int x = u / NY, yy = u - x * NY;
+                    const bool isr = yy < NR;
+                    const double *t = kt + (isr ? 2 * x * NRS + yy * NS : (2 * x + 1) * NRS + yy - NR);
+                    double acc = 0.0;
+                    if (NS == NR || isr) {
+                        const int st = isr ? 1 : NS;
+#pragma unroll
+                        for (int k = 0; k < NS; ++k) acc += t[k * st];
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < NR; ++k) acc += t[k * NS];
+                    }
+                    const int row = x < NP ? fp + x : fq + x - NP, col = isr ? fr + yy : fs + yy - NR;
+                    unsafeAtomicAdd(&b.Y[(size_t)row * ld + col], f * acc);
+                }
+            }
+            if (live && tl == 0) {
+                ++nq;
+                npq += (unsigned long long)np;
+            }
+            wave_lds_sync();
+        }
+    }
+    // the bra pair's J block: W added over the teams (lanes with the same row), then
+    // transferred once, by one lane
+#pragma unroll
+    for (int m = 0; m < C::EP; ++m) {
+#pragma unroll
+        for (int off = 32; off >= S; off >>= 1) W[m] += __shfl_xor(W[m], off, 64);
+        if (team == 0 && tl + S * m < NE) Lbra[tl + S * m] = W[m];
+    }
+    wave_lds_sync();
+    if (lane == 0) {
+        double v[NE], J[NPQ];
+#pragma unroll
+        for (int e = 0; e < NE; ++e) v[e] = Lbra[e];
+        C::B::hrr(v, ldc(a.pr.AB + 3 * b.sb), ldc(a.pr.AB + 3 * b.sb + 1), ldc(a.pr.AB + 3 * b.sb + 2), J);
+#pragma unroll
+        for (int pq = 0; pq < NPQ; ++pq) Lbra[pq] = J[pq];
+    }
+    wave_lds_sync();
+    for (int t = lane; t < NPQ; t += 64)
+        if (Lbra[t] != 0.0) unsafeAtomicAdd(&b.X[(size_t)(fp + t / NQ) * ld + fq + t % NQ], Lbra[t]);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        nq += __shfl_xor(nq, off, 64);
+        npq += __shfl_xor(npq, off, 64);
+    }
+    if (lane == 0 && nq) {
+        atomicAdd(&a.counters[3 * a.counter_slot + 0], nq);
+        atomicAdd(&a.counters[3 * a.counter_slot + 1], npq);
+        if (F32) atomicAdd(&a.counters[3 * a.counter_slot + 2], nq);
+    }
+    wave_lds_sync();  // LDS is reused by the work-group's next bra pair
+}
+
+// Wavefront form: a part's grid is (gx, gy); its work-group (x, y), number y * gx + x, takes
+// bra pairs x, x + gx, ... and, of each, the ket chunks y, y + gy, ...
+template <int LP, int LQ, int LR, int LS>
+struct WaveShared {
+    using C = WaveCfg<LP, LQ, LR, LS>;
+    WaveLDS<LP, LQ, LR, LS> team[C::TEAMS];
+    double bra[C::NPQ > C::NE ? C::NPQ : C::NE];
+};
+template <int LP, int LQ, int LR, int LS, typename R>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void jk_wave_kernel(JKLaunch J)
+{
+    __shared__ WaveShared<LP, LQ, LR, LS> L;
+    JKArgs a = J.a;
+    int gx, gy;
+    const int wg = take_part(J, a, gx, gy), x = wg % gx, y = wg / gx;
+    for (int bi = x; bi < a.n_bra; bi += gx) wave_bra<LP, LQ, LR, LS, R>(a, bi, y, gy, L.team, L.bra);
+}
+
+template <int LP, int LQ>
+__global__ __launch_bounds__(64) void schwarz_wave_kernel(DevPairs pr, DevPrims pm, int start, int n,
+                                                         double *maxI, int sph)
+{
+    using C = WaveCfg<LP, LQ, LP, LQ>;
+    constexpr int NPQ = C::NPQ, S = C::S;
+    __shared__ WaveShared<LP, LQ, LP, LQ> L;
+    const int team = threadIdx.x / S, tl = threadIdx.x - team * S;
+    const int i = blockIdx.x * C::TEAMS + team, s = start + (i < n ? i : 0);
+    const PairView v = make_view(pr, pm, s, false);
+    const int np = i < n ? v.n * v.n : 0;
+    int npmax = np;
+#pragma unroll
+    for (int off = 32; off >= S; off >>= 1) npmax = max(npmax, __shfl_xor(npmax, off, 64));
+    auto &B = L.team[team].u.d;
+    int rows[C::EP];
+    row_offsets<LP, LQ, LP, LQ>(tl, rows);
+    wave_rows<LP, LQ, LP, LQ, double>(pm, v, v, rows, B, tl, i < n, np, npmax, [](int, const double(&)[NPQ]) {});
+    double m = 0.0;
+    double *const sum = L.team[team].Prs;  // NPQ values
+#pragma unroll 1
+    for (int c0 = 0; c0 < NPQ; c0 += S) {
+        const int c = c0 + tl;
+        const bool own = i < n && c < NPQ;
+        double I[NPQ];
+#pragma unroll
+        for (int pq = 0; pq < NPQ; ++pq) I[pq] = 0.0;
+        if (own) wave_column<LP, LQ, LP, LQ, double>(v, B, c, I);
+        if (sph && (LP >= 2 || LQ >= 2)) {
+            // spherical basis: the diagonal of the solid-harmonic block, summed over columns
+            for (int ab = 0; ab < nsph(LP) * nsph(LQ); ++ab) {
+                const int al = ab / nsph(LQ), be = ab - al * nsph(LQ);
+                double y = 0.0;
+#pragma unroll
+                for (int pq = 0; pq < NPQ; ++pq) y += sph_t(LP, pq / C::NQ, al) * sph_t(LQ, pq % C::NQ, be) * I[pq];
+                y *= own ? sph_t(LP, c / C::NQ, al) * sph_t(LQ, c % C::NQ, be) : 0.0;
+#pragma unroll
+                for (int off = S / 2; off > 0; off >>= 1) y += __shfl_xor(y, off, 64);
+                if (tl == 0) sum[ab] = (c0 ? sum[ab] : 0.0) + y;
+            }
+        } else {
+#pragma unroll
+            for (int pq = 0; pq < NPQ; ++pq)
+                if (own && pq == c) m = fmax(m, fabs(I[pq]));
+        }
+    }
+    if (sph && (LP >= 2 || LQ >= 2)) {
+        wave_lds_sync();
+        for (int t = tl; t < nsph(LP) * nsph(LQ); t += S) m = fmax(m, fabs(sum[t]));
+    }
+#pragma unroll
+    for (int off = S / 2; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
+    if (tl == 0 && i < n) maxI[s] = sqrt(m);
+}
+}  // namespace rows_form
+
+namespace level_form {
+// ----------------------------------------------------------------------------------
+// Wavefront form of the classes with f shells: one 64-lane wavefront (= one work-group) on 1,
+// 2 or 4 quartets, in level order through LDS.
+// Per primitive quartet, lanes (axis, root) build the 2-D Rys tables into LDS and every
+// lane accumulates its slice of the (e0|f0) entries in registers; the ket-side and then
+// the bra-side transfer relation run level by level in LDS with lanes over entries;
+// the digestion gives each J/K target element to one lane (one atomic per element).
+// ----------------------------------------------------------------------------------
 
 // LDS budget of the wavefront form.  A class whose transfer buffers would take more keeps
 // them in a global workspace slot instead (one slot per resident work-group, persistent
@@ -1187,12 +1693,6 @@ __device__ const R *wave_eri(const DevPrims &pm, const PairView &bra, const Pair
     return src;
 }
 
-// index of the (k+1)-th set bit of m (64 if there is none)
-__device__ __forceinline__ int nth_set_bit(unsigned long long m, int k)
-{
-    for (int i = 0; i < k && m; ++i) m &= m - 1;
-    return m ? __builtin_ctzll(m) : 64;
-}
 
 // J and K digestion of one quartet's integrals I ([pq][rs], type R) by the S lanes of its
 // team: one atomic per target element; the bra-pair J block accumulates in Jpq
@@ -1446,6 +1946,7 @@ __global__ __launch_bounds__(64) void schwarz_wave_kernel(DevPairs pr, DevPrims 
         __syncthreads();
     }
 }
+}  // namespace level_form
 
 // Launchers defined in the per-class translation units (jk_class.hip).  variant 0: one
 // lane per quartet (light classes only); variant 1: one wavefront per quartet.
