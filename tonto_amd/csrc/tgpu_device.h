@@ -447,6 +447,7 @@ __device__ __forceinline__ int acc_copy()
 // Everything a wavefront needs about its bra pair, and the Schwarz frontier of its kets.
 struct BraInfo {
     int sb, tb, bp, bq, atp, atq, fp, fq, ld, kb, jend;
+    bool no_skip_prims;  // every primitive pair of the bra is below the pair cutoff
     double mIb, Pmax_b, IP_max;
     const double *P, *Pmax, *maxI;
     double *X, *Y;
@@ -455,8 +456,9 @@ struct BraInfo {
 __device__ __forceinline__ void load_bra(const JKArgs &a, int i, BraInfo &b)
 {
     b.sb = a.bra_start + i;
-    const int4 r0 = ldc(a.pr.rec0 + b.sb);
-    const int m = ldc(a.pr.rec1 + b.sb).w;
+    const int4 r0 = ldc(a.pr.rec0 + b.sb), r1 = ldc(a.pr.rec1 + b.sb);
+    const int m = r1.w;
+    b.no_skip_prims = lo16(r1.z) == 0;
     b.kb = ldc(a.ml.seg_start + m * TGPU_NBIN + a.ket_bin);
     const int kn = ldc(a.ml.seg_count + m * TGPU_NBIN + a.ket_bin);
     const int jlim = a.same_bin ? b.sb - ldc(a.ml.seg_start + m * TGPU_NBIN + a.bra_bin) + 1 : kn;
@@ -496,6 +498,7 @@ __device__ __forceinline__ void load_bra(const JKArgs &a, int i, BraInfo &b)
 struct KetTest {
     int sk, fr, fs;
     bool skipJ, skipK, skip_lists;
+    bool empty;    // no primitive quartet: every primitive pair of bra or ket dropped
     int halvings;  // permutation factor f = 2^-halvings
     double f;
 };
@@ -540,6 +543,10 @@ __device__ __forceinline__ bool test_ket(const JKArgs &a, const BraInfo &b, int 
     const bool any_same = b.atp == b.atq || akr == aks || b.atp == akr || b.atp == aks ||
                           b.atq == akr || b.atq == aks;
     t.skip_lists = !any_same;
+    // Of a quartet over four distinct atoms the primitive pairs below the pair cutoff are
+    // dropped; where that leaves a pair without any, the integrals are exactly zero.  Such
+    // quartets are counted and not computed.
+    t.empty = t.skip_lists && (b.no_skip_prims || lo16(ldc(a.pr.rec1 + t.sk).z) == 0);
     return true;
 }
 
@@ -840,7 +847,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
         if (j0 < b.jend) {
             const int j = j0 + lane;
             KetTest t;
-            const bool ok = j < b.jend && test_ket(a, b, j, t, pmr, nsh);
+            bool ok = j < b.jend && test_ket(a, b, j, t, pmr, nsh);
+            if (ok && t.empty) {
+                ok = false;
+                ++nq;
+                if (MIXED && j >= jsplit) ++n32;
+            }
             const unsigned long long m = __ballot(ok);
             if (ok) {
                 const int pos = qn + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
@@ -874,7 +886,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
     for (int j0 = KROWS ? 64 * wave : 0; j0 < b.jend; j0 += KROWS ? 256 : 64) {
         const int j = j0 + lane;
         KetTest t;
-        if (j < b.jend && test_ket(a, b, j, t, pmr, nsh))
+        const bool ok = j < b.jend && test_ket(a, b, j, t, pmr, nsh);
+        if (ok && t.empty) {
+            ++nq;
+            if (MIXED && j >= jsplit) ++n32;
+        } else if (ok)
             quartet(j, (int)t.skipJ | ((int)t.skipK << 1) | ((int)t.skip_lists << 2) | (t.halvings << 3),
                     t.fr, t.fs, make_view(a.pr, a.pm, b.sb, t.skip_lists), 0, 0);
     }
@@ -1208,7 +1224,11 @@ __device__ void wave_bra(const JKArgs &a, int bi, int y, int gy, WaveLDS<LP, LQ,
     for (int jc = jbeg + y * a.ket_chunk; jc < jend; jc += step) {
         const int jlim = min(jend, jc + a.ket_chunk);
         KetTest tt;
-        const bool ok = jc + lane < jlim && test_ket(a, b, jc + lane, tt);
+        bool ok = jc + lane < jlim && test_ket(a, b, jc + lane, tt);
+        if (ok && tt.empty) {
+            ok = false;
+            ++nq;
+        }
         const int flags_l = ok ? ((int)tt.skipJ | ((int)tt.skipK << 1) | ((int)tt.skip_lists << 2) |
                                   (tt.halvings << 3))
                                : 0;
@@ -1813,7 +1833,11 @@ __device__ void wave_bra(const JKArgs &a, int bi, int y, int gy, WaveLDS<LP, LQ,
     for (int jc = jbeg + y * a.ket_chunk; jc < jend; jc += step) {
         const int jlim = min(jend, jc + a.ket_chunk);
         KetTest tt;
-        const bool ok = jc + lane < jlim && test_ket(a, b, jc + lane, tt);
+        bool ok = jc + lane < jlim && test_ket(a, b, jc + lane, tt);
+        if (ok && tt.empty) {
+            ok = false;
+            ++nq;
+        }
         const int flags_l = ok ? ((int)tt.skipJ | ((int)tt.skipK << 1) | ((int)tt.skip_lists << 2) |
                                   (tt.halvings << 3))
                                : 0;
