@@ -1,13 +1,14 @@
 // Training and inference kernels of the learned initial guess's network (FP32).
 //
-// Every dense-layer product, forward and backward, is one LDS-tiled GEMM kernel with
-// general strides (so X^T dZ and dZ W^T read their operands in place, no transposed
-// copies): 64 x 64 output tile per 256-lane work-group, 4 x 4 per lane, K in steps of
-// 16 through LDS.  The forward epilogue adds the bias, keeps the pre-activation and
-// applies SiLU; the weight-gradient product splits its long K (= rows of the batch)
-// over blockIdx.z and accumulates with atomics.  FP32 MFMA gives no more than the
-// MI355X's FP32 vector rate (157.3 TFLOP/s each), and these products are small next to
-// the J/K builds, so the kernel stays on the vector ALU.
+// The products run on the matrix cores (v_mfma_f32_16x16x4f32: FP32 operands, products and
+// sums, twice the vector rate without packed FP32), and what bounded the step were its 16
+// launches in series, most on 64 work-groups: a 2048-row step of the 273-128-128-225 network
+// took 727 us for 0.85 GFLOP.  Now a forward pass is one launch and a backward pass two:
+//   forward  16 rows per work-group through all three layers, activations in LDS;
+//   chain    16 rows per work-group: dZ2 = (dY W3^T) SiLU'(Z2), dZ1 = (dZ2 W2^T) SiLU'(Z1);
+//   weights  32 x 32 tiles of dW1, dW2, dW3 (and the bias sums), eight wavefronts sharing the
+//            batch's rows and adding up in LDS: no atomics up to 16384 rows.
+// Networks whose 16-row block does not fit the LDS use a general tiled product per layer.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -25,11 +26,10 @@ struct GemmArgs {
     float *C;
     long scm;       // C(m, n) = C[m * scm + n]
     long M;
-    int N, K, kchunk;
+    int N, K;
     const float *bias;  // added per column (forward epilogue), or null
     float *Z;           // pre-activation copy (ld scm), or null
     int act;            // 1: SiLU
-    int atomic;         // accumulate into C with atomics (split-K; no bias / act)
 };
 
 __device__ __forceinline__ float silu(float z) { return z / (1.0f + expf(-z)); }
@@ -49,8 +49,6 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g)
     const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
     const long m0 = (long)blockIdx.y * TM;
     const int n0 = blockIdx.x * TN;
-    const int k_begin = blockIdx.z * g.kchunk;
-    const int k_end = min(g.K, k_begin + g.kchunk);
     float acc[4][4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -58,17 +56,17 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g)
         for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
     // lanes walk the unit-stride index of each operand, so tile loads are coalesced
     const bool a_m_fast = g.sam == 1, b_n_fast = g.sbn == 1;
-    for (int k0 = k_begin; k0 < k_end; k0 += TK) {
+    for (int k0 = 0; k0 < g.K; k0 += TK) {
         for (int t = threadIdx.x; t < TM * TK; t += 256) {
             const int mm = a_m_fast ? t % TM : t / TK, kk = a_m_fast ? t / TM : t % TK;
             const long m = m0 + mm;
             const int k = k0 + kk;
-            As[kk][mm] = (m < g.M && k < k_end) ? g.A[m * g.sam + (long)k * g.sak] : 0.0f;
+            As[kk][mm] = (m < g.M && k < g.K) ? g.A[m * g.sam + (long)k * g.sak] : 0.0f;
         }
         for (int t = threadIdx.x; t < TN * TK; t += 256) {
             const int nn = b_n_fast ? t % TN : t / TK, kk = b_n_fast ? t / TN : t % TK;
             const int n = n0 + nn, k = k0 + kk;
-            Bs[kk][nn] = (n < g.N && k < k_end) ? g.B[(long)k * g.sbk + (long)n * g.sbn] : 0.0f;
+            Bs[kk][nn] = (n < g.N && k < g.K) ? g.B[(long)k * g.sbk + (long)n * g.sbn] : 0.0f;
         }
         __syncthreads();
 #pragma unroll
@@ -94,10 +92,6 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g)
             const int n = n0 + tx * 4 + j;
             if (n >= g.N) continue;
             float v = acc[i][j];
-            if (g.atomic) {
-                atomicAdd(&g.C[m * g.scm + n], v);
-                continue;
-            }
             if (g.bias) v += g.bias[n];
             if (g.Z) g.Z[m * g.scm + n] = v;
             if (g.act) v = silu(v);
@@ -108,20 +102,9 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g)
 
 void gemm(const GemmArgs &g0, hipStream_t s)
 {
-    GemmArgs g = g0;
-    const long mt = (g.M + TM - 1) / TM;
-    const int nt = (g.N + TN - 1) / TN;
-    int kz = 1;
-    if (g.atomic) {
-        // split K so that the grid has about 2048 work-groups
-        const long want = std::max(1L, 2048 / std::max(1L, mt * nt));
-        kz = (int)std::min<long>(want, (g.K + 255) / 256);
-        if (kz < 1) kz = 1;
-    }
-    g.kchunk = ((g.K + kz - 1) / kz + TK - 1) / TK * TK;
-    kz = (g.K + g.kchunk - 1) / g.kchunk;
-    if (kz < 1) kz = 1;
-    gemm_kernel<<<dim3(nt, (unsigned)mt, kz), 256, 0, s>>>(g);
+    const long mt = (g0.M + TM - 1) / TM;
+    const int nt = (g0.N + TN - 1) / TN;
+    gemm_kernel<<<dim3(nt, (unsigned)mt), 256, 0, s>>>(g0);
 }
 
 __global__ void fill_kernel(float *p, long n, float v)
@@ -129,22 +112,11 @@ __global__ void fill_kernel(float *p, long n, float v)
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = v;
 }
 
-// dZ = dA * SiLU'(Z)
-__global__ void silu_back_kernel(const float *dA, const float *Z, float *dZ, long n)
+// d = d * SiLU'(Z)
+__global__ void silu_back_kernel(float *d, const float *Z, long n)
 {
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-        dZ[i] = dA[i] * silu_grad(Z[i]);
-}
-
-// db[n] += sum over this work-group's rows of dZ[m][n] (blockDim.x >= N)
-__global__ void colsum_kernel(const float *dZ, long M, int N, int rows, float *db)
-{
-    const int n = threadIdx.x;
-    if (n >= N) return;
-    const long r0 = (long)blockIdx.x * rows, r1 = min(M, r0 + rows);
-    float acc = 0.0f;
-    for (long m = r0; m < r1; ++m) acc += dZ[m * N + n];
-    atomicAdd(&db[n], acc);
+        d[i] *= silu_grad(Z[i]);
 }
 
 __global__ __launch_bounds__(256) void mse_kernel(const float *Y, const float *T, long n, float scale,
@@ -176,6 +148,209 @@ __global__ void adam_kernel(float *p, const float *g, float *m, float *v, long n
         m[i] = mi;
         v[i] = vi;
         p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    }
+}
+
+// ----------------------------------------------------------------------------------------
+// Matrix-core form.  v_mfma_f32_16x16x4f32: lane l gives A(l % 16, l / 16) and B(l / 16, l % 16)
+// and holds C(4 (l / 16) + i, l % 16), i = 0 .. 3.
+// ----------------------------------------------------------------------------------------
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+constexpr int kRows = 16;    // batch rows of a work-group
+constexpr int kWaves = 8;    // wavefronts of a work-group
+constexpr int kUnroll = 8;   // k steps (of 4) whose loads are in flight together
+constexpr size_t kLdsLimit = 64 * 1024;
+
+// LDS row of K values: zero-padded to whole unrolled steps, odd length (bank spread)
+__host__ __device__ constexpr int lds_stride(int K) { return (K + 4 * kUnroll - 1) / (4 * kUnroll) * (4 * kUnroll) + 1; }
+
+// rows m0 .. of the M x K matrix src into LDS (row stride lds_stride(K)), zeros elsewhere
+__device__ __forceinline__ void stage_rows(const float *src, long m0, long M, int K, float *dst)
+{
+    const int s = lds_stride(K);
+    for (int t = threadIdx.x; t < kRows * s; t += blockDim.x) {
+        const int r = t / s, k = t - r * s;
+        dst[t] = k < K && m0 + r < M ? src[(m0 + r) * K + k] : 0.0f;
+    }
+}
+
+// C = A B for the 16 rows in LDS (As, K columns) and the N columns of B, B(k, n) =
+// W[k * sk + n * sn]; done(row, n, value) is called for every element with n < N.
+template <typename Done>
+__device__ __forceinline__ void rows_product(const float *As, int K, const float *W, long sk, long sn, int N, Done &&done)
+{
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    const int sa = lds_stride(K);
+    for (int t = threadIdx.x >> 6; t * 16 < N; t += kWaves) {
+        const int n = t * 16 + c;
+        const bool in = n < N;
+        const float *w = W + (long)(in ? n : 0) * sn;
+        f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int k0 = 0; k0 < K; k0 += 4 * kUnroll) {
+            float a[kUnroll], b[kUnroll];
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) {
+                const int k = k0 + 4 * u + g;
+                a[u] = As[c * sa + k];
+                b[u] = in && k < K ? w[(long)k * sk] : 0.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b[u], acc, 0, 0, 0);
+        }
+        if (in) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) done(4 * g + i, n, acc[i]);
+        }
+    }
+}
+
+// zero padding of an LDS block whose first N columns rows_product fills
+__device__ __forceinline__ void zero_pad(float *dst, int N)
+{
+    const int s = lds_stride(N), w = s - N;
+    for (int t = threadIdx.x; t < kRows * w; t += blockDim.x) dst[t / w * s + N + t % w] = 0.0f;
+}
+
+struct NetArgs {
+    const float *W1, *b1, *W2, *b2, *W3, *b3;
+    int n_in, nh, n_out;
+    long M;
+};
+
+__host__ __device__ constexpr size_t forward_lds(int n_in, int nh) { return 4u * kRows * ((size_t)lds_stride(n_in) + lds_stride(nh)); }
+__host__ __device__ constexpr size_t chain_lds(int nh, int n_out) { return 4u * kRows * ((size_t)lds_stride(n_out) + lds_stride(nh)); }
+
+__global__ __launch_bounds__(64 * kWaves) void forward_kernel(NetArgs a, const float *X, float *Z1, float *A1, float *Z2,
+                                                             float *A2, float *Y)
+{
+    extern __shared__ float sm[];
+    float *const u = sm, *const v = sm + kRows * (lds_stride(a.n_in) > lds_stride(a.nh) ? lds_stride(a.n_in) : lds_stride(a.nh));
+    const long m0 = (long)blockIdx.x * kRows;
+    const int sh = lds_stride(a.nh);
+    stage_rows(X, m0, a.M, a.n_in, u);
+    zero_pad(v, a.nh);
+    __syncthreads();
+    // one hidden layer: pre-activation and activation out, the activation into LDS too
+    auto hidden = [&](const float *b, float *Z, float *A, float *next, int r, int n, float x) {
+        const float z = x + b[n], y = silu(z);
+        next[r * sh + n] = y;
+        if (m0 + r < a.M) {
+            Z[(m0 + r) * a.nh + n] = z;
+            A[(m0 + r) * a.nh + n] = y;
+        }
+    };
+    rows_product(u, a.n_in, a.W1, a.nh, 1, a.nh, [&](int r, int n, float x) { hidden(a.b1, Z1, A1, v, r, n, x); });
+    __syncthreads();
+    zero_pad(u, a.nh);  // (u held X)
+    rows_product(v, a.nh, a.W2, a.nh, 1, a.nh, [&](int r, int n, float x) { hidden(a.b2, Z2, A2, u, r, n, x); });
+    __syncthreads();
+    rows_product(u, a.nh, a.W3, a.n_out, 1, a.n_out, [&](int r, int n, float x) {
+        if (m0 + r < a.M) Y[(m0 + r) * a.n_out + n] = x + a.b3[n];
+    });
+}
+
+__global__ __launch_bounds__(64 * kWaves) void chain_kernel(NetArgs a, const float *Z1, const float *Z2, const float *dY,
+                                                           float *dZ1, float *dZ2)
+{
+    extern __shared__ float sm[];
+    float *const u = sm, *const v = sm + kRows * lds_stride(a.n_out);
+    const long m0 = (long)blockIdx.x * kRows;
+    const int sh = lds_stride(a.nh);
+    stage_rows(dY, m0, a.M, a.n_out, u);
+    zero_pad(v, a.nh);
+    __syncthreads();
+    rows_product(u, a.n_out, a.W3, 1, a.n_out, a.nh, [&](int r, int n, float x) {
+        const bool in = m0 + r < a.M;
+        const float d = in ? x * silu_grad(Z2[(m0 + r) * a.nh + n]) : 0.0f;
+        v[r * sh + n] = d;
+        if (in) dZ2[(m0 + r) * a.nh + n] = d;
+    });
+    __syncthreads();
+    rows_product(v, a.nh, a.W2, 1, a.nh, a.nh, [&](int r, int n, float x) {
+        if (m0 + r < a.M) dZ1[(m0 + r) * a.nh + n] = x * silu_grad(Z1[(m0 + r) * a.nh + n]);
+    });
+}
+
+// C(m, n) = sum over the batch of A(r, m) B(r, n), c(n) = sum of B(r, n), three such products;
+// a 32 x 32 tile per work-group, the batch's rows shared by its wavefronts (and by gridDim.y
+// work-groups, which then add with atomics).
+struct GradProduct {
+    const float *A, *B;
+    float *C, *c;
+    int m, n;       // columns of A and of B
+    int tn, first;  // tiles along n, first work-group
+};
+struct GradArgs {
+    GradProduct p[3];
+    long M;
+    long rows;  // batch rows per blockIdx.y, a multiple of 4 kWaves
+};
+
+__global__ __launch_bounds__(64 * kWaves) void grad_kernel(GradArgs g)
+{
+    __shared__ float part[kWaves][32 * 32];
+    __shared__ float cpart[kWaves][32];
+    const int wg = blockIdx.x;
+    const int q = wg >= g.p[2].first ? 2 : wg >= g.p[1].first ? 1 : 0;
+    const GradProduct p = g.p[q];
+    const int tile = wg - p.first, m0 = tile / p.tn * 32, n0 = tile % p.tn * 32;
+    const int lane = threadIdx.x & 63, c = lane & 15, k = lane >> 4, wave = threadIdx.x >> 6;
+    const long r_begin = (long)blockIdx.y * g.rows, r_end = min(g.M, r_begin + g.rows);
+    const bool ma = m0 + c < p.m, mb = m0 + 16 + c < p.m, na = n0 + c < p.n, nb = n0 + 16 + c < p.n;
+    f4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    float cs[2] = {0.0f, 0.0f};
+    constexpr int U = 4;
+    for (long r0 = r_begin + 4 * U * wave; r0 < r_end; r0 += 4 * U * kWaves) {
+        float a[U][2], b[U][2];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const long r = r0 + 4 * u + k;
+            const bool in = r < r_end;
+            const float *ar = p.A + (in ? r : 0) * p.m + m0 + c, *br = p.B + (in ? r : 0) * p.n + n0 + c;
+            a[u][0] = in && ma ? ar[0] : 0.0f;
+            a[u][1] = in && mb ? ar[16] : 0.0f;
+            b[u][0] = in && na ? br[0] : 0.0f;
+            b[u][1] = in && nb ? br[16] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i], b[u][j], acc[i][j], 0, 0, 0);
+            cs[0] += b[u][0];
+            cs[1] += b[u][1];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[wave][(16 * i + 4 * k + e) * 32 + 16 * j + c] = acc[i][j][e];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        cs[j] += __shfl_xor(cs[j], 16, 64);
+        cs[j] += __shfl_xor(cs[j], 32, 64);
+        if (k == 0) cpart[wave][16 * j + c] = cs[j];
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < 32 * 32 + 32; t += 64 * kWaves) {
+        const bool bias = t >= 32 * 32;
+        const int m = m0 + t / 32, n = n0 + t % 32;
+        if (n >= p.n || (bias ? m0 > 0 : m >= p.m)) continue;
+        float v = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) v += bias ? cpart[w][t % 32] : part[w][t];
+        float *dst = bias ? p.c + n : p.C + (long)m * p.n + n;
+        if (gridDim.y > 1) atomicAdd(dst, v);
+        else *dst = v;
     }
 }
 
@@ -223,11 +398,17 @@ extern "C" int tmlp_forward(const float *params, int n_in, int nh, int n_out, co
     hipStream_t s = (hipStream_t)stream;
     const Layout L = layout(n_in, nh, n_out);
     float *Z1 = ws, *A1 = ws + M * nh, *Z2 = ws + 2 * M * nh, *A2 = ws + 3 * M * nh;
+    const size_t lds = forward_lds(std::max(n_in, nh), nh);
+    if (lds <= kLdsLimit) {
+        const NetArgs a{params + L.W1, params + L.b1, params + L.W2, params + L.b2, params + L.W3, params + L.b3, n_in, nh, n_out, M};
+        forward_kernel<<<(unsigned)((M + kRows - 1) / kRows), 64 * kWaves, lds, s>>>(a, X, Z1, A1, Z2, A2, Y);
+        return hipGetLastError() == hipSuccess ? TMLP_OK : TMLP_E_HIP;
+    }
     GemmArgs g{};
     g.A = X; g.sam = n_in; g.sak = 1;
     g.B = params + L.W1; g.sbk = nh; g.sbn = 1;
     g.C = A1; g.scm = nh; g.M = M; g.N = nh; g.K = n_in;
-    g.bias = params + L.b1; g.Z = Z1; g.act = 1; g.atomic = 0;
+    g.bias = params + L.b1; g.Z = Z1; g.act = 1;
     gemm(g, s);
     g.A = A1; g.sam = nh;
     g.B = params + L.W2; g.sbk = nh;
@@ -246,45 +427,44 @@ extern "C" int tmlp_backward(const float *params, int n_in, int nh, int n_out, c
     if (!params || !X || !ws || !dY || !grads || !ws2 || bad_dims(n_in, nh, n_out, M)) return TMLP_E_ARG;
     hipStream_t s = (hipStream_t)stream;
     const Layout L = layout(n_in, nh, n_out);
-    fill_kernel<<<grid_1d(L.n), 256, 0, s>>>(grads, L.n, 0.0f);
+    const long rows_step = 4 * kWaves;
+    // one work-group per tile and 16384 rows
+    const int kz = (int)std::max(1L, (M + 16383) / 16384);
+    if (kz > 1 || M == 0) fill_kernel<<<grid_1d(L.n), 256, 0, s>>>(grads, L.n, 0.0f);
     if (M == 0) return hipGetLastError() == hipSuccess ? TMLP_OK : TMLP_E_HIP;
     const float *Z1 = ws, *A1 = ws + M * nh, *Z2 = ws + 2 * M * nh, *A2 = ws + 3 * M * nh;
-    float *dA = ws2, *dZ = ws2 + M * nh;
-    const int rows = 512;
-    const unsigned cs_grid = (unsigned)((M + rows - 1) / rows);
-    GemmArgs g{};
-    // layer 3: dW3 = A2^T dY, db3 = colsum dY, dA2 = dY W3^T
-    g.A = A2; g.sam = 1; g.sak = nh;
-    g.B = dY; g.sbk = n_out; g.sbn = 1;
-    g.C = grads + L.W3; g.scm = n_out; g.M = nh; g.N = n_out; g.K = (int)M; g.atomic = 1;
-    gemm(g, s);
-    colsum_kernel<<<cs_grid, std::max(64, (n_out + 63) / 64 * 64), 0, s>>>(dY, M, n_out, rows, grads + L.b3);
-    g = GemmArgs{};
-    g.A = dY; g.sam = n_out; g.sak = 1;
-    g.B = params + L.W3; g.sbk = 1; g.sbn = n_out;
-    g.C = dA; g.scm = nh; g.M = M; g.N = nh; g.K = n_out;
-    gemm(g, s);
-    silu_back_kernel<<<grid_1d(M * nh), 256, 0, s>>>(dA, Z2, dZ, M * nh);
-    // layer 2: dW2 = A1^T dZ2, db2, dA1 = dZ2 W2^T
-    g = GemmArgs{};
-    g.A = A1; g.sam = 1; g.sak = nh;
-    g.B = dZ; g.sbk = nh; g.sbn = 1;
-    g.C = grads + L.W2; g.scm = nh; g.M = nh; g.N = nh; g.K = (int)M; g.atomic = 1;
-    gemm(g, s);
-    colsum_kernel<<<cs_grid, std::max(64, (nh + 63) / 64 * 64), 0, s>>>(dZ, M, nh, rows, grads + L.b2);
-    g = GemmArgs{};
-    g.A = dZ; g.sam = nh; g.sak = 1;
-    g.B = params + L.W2; g.sbk = 1; g.sbn = nh;
-    g.C = dA; g.scm = nh; g.M = M; g.N = nh; g.K = nh;
-    gemm(g, s);
-    silu_back_kernel<<<grid_1d(M * nh), 256, 0, s>>>(dA, Z1, dZ, M * nh);
-    // layer 1: dW1 = X^T dZ1, db1
-    g = GemmArgs{};
-    g.A = X; g.sam = 1; g.sak = n_in;
-    g.B = dZ; g.sbk = nh; g.sbn = 1;
-    g.C = grads + L.W1; g.scm = nh; g.M = n_in; g.N = nh; g.K = (int)M; g.atomic = 1;
-    gemm(g, s);
-    colsum_kernel<<<cs_grid, std::max(64, (nh + 63) / 64 * 64), 0, s>>>(dZ, M, nh, rows, grads + L.b1);
+    float *dZ1 = ws2, *dZ2 = ws2 + M * nh;
+    const size_t lds = chain_lds(nh, n_out);
+    if (lds <= kLdsLimit) {
+        const NetArgs a{params + L.W1, params + L.b1, params + L.W2, params + L.b2, params + L.W3, params + L.b3, n_in, nh, n_out, M};
+        chain_kernel<<<(unsigned)((M + kRows - 1) / kRows), 64 * kWaves, lds, s>>>(a, Z1, Z2, dY, dZ1, dZ2);
+    } else {
+        // dA2 = dY W3^T and dA1 = dZ2 W2^T by the general product, SiLU' in place
+        GemmArgs g{};
+        g.A = dY; g.sam = n_out; g.sak = 1;
+        g.B = params + L.W3; g.sbk = 1; g.sbn = n_out;
+        g.C = dZ2; g.scm = nh; g.M = M; g.N = nh; g.K = n_out;
+        gemm(g, s);
+        silu_back_kernel<<<grid_1d(M * nh), 256, 0, s>>>(dZ2, Z2, M * nh);
+        g.A = dZ2; g.sam = nh;
+        g.B = params + L.W2; g.sbn = nh;
+        g.C = dZ1; g.K = nh;
+        gemm(g, s);
+        silu_back_kernel<<<grid_1d(M * nh), 256, 0, s>>>(dZ1, Z1, M * nh);
+    }
+    GradArgs g{};
+    g.p[0] = GradProduct{X, dZ1, grads + L.W1, grads + L.b1, n_in, nh, 0, 0};
+    g.p[1] = GradProduct{A1, dZ2, grads + L.W2, grads + L.b2, nh, nh, 0, 0};
+    g.p[2] = GradProduct{A2, dY, grads + L.W3, grads + L.b3, nh, n_out, 0, 0};
+    long tiles = 0;
+    for (GradProduct &p : g.p) {
+        p.tn = (p.n + 31) / 32;
+        p.first = (int)tiles;
+        tiles += (long)((p.m + 31) / 32) * p.tn;
+    }
+    g.M = M;
+    g.rows = ((M + kz - 1) / kz + rows_step - 1) / rows_step * rows_step;
+    grad_kernel<<<dim3((unsigned)tiles, (unsigned)kz), 64 * kWaves, 0, s>>>(g);
     return hipGetLastError() == hipSuccess ? TMLP_OK : TMLP_E_HIP;
 }
 
