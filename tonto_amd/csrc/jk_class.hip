@@ -47,9 +47,13 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, cons
         static bool attr_set = false;
         if (!attr_set) {
             // dynamic LDS above the 64 KiB default has to be allowed per kernel
-            (void)hipFuncSetAttribute((const void *)jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, true>,
+            (void)hipFuncSetAttribute((const void *)jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, KR_GROUP>,
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kMaxLds - kStatic));
-            (void)hipFuncSetAttribute((const void *)jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, true>,
+            (void)hipFuncSetAttribute((const void *)jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, KR_GROUP>,
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kMaxLds - kStatic));
+            (void)hipFuncSetAttribute((const void *)jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, KR_WAVE>,
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kMaxLds - kStatic));
+            (void)hipFuncSetAttribute((const void *)jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, KR_WAVE>,
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kMaxLds - kStatic));
             attr_set = true;
         }
@@ -95,13 +99,37 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, cons
         }
 #if !(TGPU_LP == 3 && TGPU_LQ == 3 && TGPU_LR == 0 && TGPU_LS == 0)
         if (rows_grid > 0) {
-            if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, true><<<rows_grid, 256, lds, s>>>(rows);
-            else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, true><<<rows_grid, 256, lds, s>>>(rows);
+            if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, KR_GROUP><<<rows_grid, 256, lds, s>>>(rows);
+            else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, KR_GROUP><<<rows_grid, 256, lds, s>>>(rows);
         }
 #endif
         if (glob_grid > 0) {
-            if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, false><<<glob_grid, 256, 0, s>>>(glob);
-            else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, false><<<glob_grid, 256, 0, s>>>(glob);
+            // The rows of the wavefronts' own bra pairs in LDS, at most kWaveRowsLds per work-
+            // group if all of them then fit (two work-groups per CU), else as many as fit one,
+            // down to a quarter of them; global updates only for (ff|ss) (as above), where K is
+            // not digested, and for molecules too large for a quarter.
+            size_t wlds = 0;
+#if !(TGPU_LP == 3 && TGPU_LQ == 3 && TGPU_LR == 0 && TGPU_LS == 0)
+            constexpr size_t kWaveRowsLds = 76 * 1024;
+            const size_t Wmax = a.kcol_max[TGPU_LR] + (TGPU_LR == TGPU_LS ? 0 : a.kcol_max[TGPU_LS]);
+            const size_t row4 = 4 * Wmax * sizeof(double);  // one row of each wavefront
+            const size_t room = budget > kStatic ? budget - kStatic : 0;
+            const size_t small = budget < kWaveRowsLds ? room : kWaveRowsLds - kStatic;
+            int nwr = row4 ? (int)std::min<size_t>(NP + NQ, small / row4) : 0;
+            if (nwr < NP + NQ && row4) nwr = (int)std::min<size_t>(NP + NQ, room / row4);
+            if (a.kp != HUGE_VAL && a.kcol && 4 * nwr >= NP + NQ) {
+                glob.a.krow_rows = nwr;
+                glob.a.krow_stride = (int)(nwr * Wmax);
+                wlds = nwr * row4;
+            }
+            if (wlds) {
+                if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, KR_WAVE><<<glob_grid, 256, wlds, s>>>(glob);
+                else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, KR_WAVE><<<glob_grid, 256, wlds, s>>>(glob);
+                return TGPU_OK;
+            }
+#endif
+            if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, KR_GLOBAL><<<glob_grid, 256, 0, s>>>(glob);
+            else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, KR_GLOBAL><<<glob_grid, 256, 0, s>>>(glob);
         }
         return TGPU_OK;
     }

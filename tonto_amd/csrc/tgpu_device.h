@@ -371,6 +371,12 @@ struct JKArgs {
     const int *kcol;
     const int *kcol_map;
     int kcol_lofs[TGPU_LMAX + 2];
+    // Per molecule m: its functions of momentum l are kcol_map[klofs[(TGPU_LMAX + 2) m + l]
+    // .. klofs[(TGPU_LMAX + 2) m + l + 1]).  kcol_max[l]: the most functions of momentum l of
+    // a molecule.  krow_stride: LDS doubles of one wavefront's rows (rows per wavefront).
+    const int *klofs;
+    int kcol_max[TGPU_LMAX + 1];
+    int krow_stride;
     // UHF pass: J from Tonto's ket side only, X(cd) += f (ab|cd) P(ab) with ab the pair of
     // larger Tonto index, for ab != cd (the updates Tonto's UHF engine puts into JA
     // through JBcd => JA(cd), molecule.fock.foo:2637)
@@ -446,7 +452,7 @@ __device__ __forceinline__ int acc_copy()
 
 // Everything a wavefront needs about its bra pair, and the Schwarz frontier of its kets.
 struct BraInfo {
-    int sb, tb, bp, bq, atp, atq, fp, fq, ld, kb, jend;
+    int sb, tb, bp, bq, atp, atq, fp, fq, ld, kb, jend, mol;
     bool no_skip_prims;  // every primitive pair of the bra is below the pair cutoff
     double mIb, Pmax_b, IP_max;
     const double *P, *Pmax, *maxI;
@@ -458,6 +464,7 @@ __device__ __forceinline__ void load_bra(const JKArgs &a, int i, BraInfo &b)
     b.sb = a.bra_start + i;
     const int4 r0 = ldc(a.pr.rec0 + b.sb), r1 = ldc(a.pr.rec1 + b.sb);
     const int m = r1.w;
+    b.mol = m;
     b.no_skip_prims = lo16(r1.z) == 0;
     b.kb = ldc(a.ml.seg_start + m * TGPU_NBIN + a.ket_bin);
     const int kn = ldc(a.ml.seg_count + m * TGPU_NBIN + a.ket_bin);
@@ -581,8 +588,12 @@ __device__ __forceinline__ void wave_lds_sync()
 // krow_rows x W doubles, W = the number of functions of momentum LR, plus those of
 // momentum LS if LS != LR) and are flushed once, row by row, with atomics that skip zeros;
 // the other rows are updated with global atomics.  Otherwise four bra pairs per
-// work-group, one per wavefront, and every K update is a global atomic.
-template <int LP, int LQ, int LR, int LS, bool MIXED, bool KROWS>
+// work-group, one per wavefront; each wavefront then keeps its own bra pair's rows (WROWS),
+// restricted to the columns of its molecule, where they fit and the bra pair has more K
+// updates ahead than the rows have entries.  Scattered FP64 atomics (2.5e10/s over the chip)
+// bounded every class of a batch before: (ps|ps) 81 ms, (dp|ps) 44 ms for 256 clusters.
+enum KRowsForm { KR_GLOBAL = 0, KR_GROUP = 1, KR_WAVE = 2 };
+template <int LP, int LQ, int LR, int LS, bool MIXED, int KR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_waves(LP, LQ, LR, LS), 8))) void jk_kernel(JKLaunch L)
 {
     JKArgs a = L.a;
@@ -590,6 +601,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
     const int wg = take_part(L, a, gx, gy);
     constexpr int NP = ncart(LP), NQ = ncart(LQ), NR = ncart(LR), NS = ncart(LS);
     constexpr int NPQ = NP * NQ, NRS = NR * NS, NI = NPQ * NRS;
+    constexpr bool KROWS = KR == KR_GROUP, WROWS = KR == KR_WAVE;
     constexpr int NRT = EriBody<LP, LQ, LR, LS, double>::NROOT;
     // the n-root Rys table in LDS (<= 18 KB): the root/weight lookups of every primitive
     // quartet then hit LDS instead of L2
@@ -599,7 +611,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
     // (j << 5 | flags, fr << 16 | fs); basis functions < 65536 (tgpu_create)
     __shared__ int2 kqueue[4][128];
 #endif
-    extern __shared__ double krow[];  // KROWS: [NP + NQ][ld]
+    extern __shared__ double krow_all[];  // KROWS: [NP + NQ][W]; WROWS: four times krow_stride
     const int lane = threadIdx.x & 63;
     // the bra pair is uniform over the wavefront: readfirstlane lets the compiler keep
     // everything derived from it in scalar registers
@@ -621,10 +633,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
         load_bra(a, i, b);
     }
     const int ld = b.ld, fp = b.fp, fq = b.fq;
-    const int nkr = KROWS ? a.krow_rows : 0;  // K rows accumulated in LDS
     // LDS row: the nR functions of momentum LR, then (LS != LR) those of momentum LS
-    const int nR = KROWS ? a.kcol_lofs[LR + 1] - a.kcol_lofs[LR] : 0;
-    const int W = KROWS ? (LR == LS ? nR : nR + a.kcol_lofs[LS + 1] - a.kcol_lofs[LS]) : 0;
+    const int *lofs = WROWS ? a.klofs + (TGPU_LMAX + 2) * b.mol : nullptr;
+    const int lofR = KROWS ? a.kcol_lofs[LR] : WROWS ? ldc(lofs + LR) : 0;
+    const int lofS = KROWS ? a.kcol_lofs[LS] : WROWS ? ldc(lofs + LS) : 0;
+    const int nR = KROWS ? a.kcol_lofs[LR + 1] - lofR : WROWS ? ldc(lofs + LR + 1) - lofR : 0;
+    const int nS = KROWS ? a.kcol_lofs[LS + 1] - lofS : WROWS ? ldc(lofs + LS + 1) - lofS : 0;
+    const int W = LR == LS ? nR : nR + nS;
+    constexpr int KEL = (NP + NQ) * (NR + NS);  // K elements of a quartet
+    const int nkr = KROWS ? a.krow_rows  // K rows accumulated in LDS
+                    : WROWS && (long long)b.jend * KEL > (long long)a.krow_rows * W ? a.krow_rows
+                                                                                   : 0;
+    double *const krow = WROWS ? krow_all + wave * a.krow_stride : krow_all;
     // P rows (KROWS with (ss) kets, prefixes of at least krow_min_kets kets (256 unless
     // set), when all NP + NQ rows fit): the bra pair's density rows at the same columns as its K rows, staged in LDS
     // after them, so that the K digestion reads P(bra function, ket function) from LDS,
@@ -647,15 +667,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
         for (int t = threadIdx.x; t < nkr * W; t += blockDim.x) krow[t] = 0.0;
         for (int t = threadIdx.x; PR && t < npr * W; t += blockDim.x) {
             const int row = t / W, cc = t - row * W;
-            const int col = ldc(a.kcol_map + (cc < nR ? a.kcol_lofs[LR] + cc : a.kcol_lofs[LS] + cc - nR));
+            const int col = ldc(a.kcol_map + (cc < nR ? lofR + cc : lofS + cc - nR));
             prow[t] = b.P[(size_t)(row < NP ? fp + row : fq + row - NP) * ld + col];
         }
         __syncthreads();
     }
+    if (WROWS) {
+        for (int t = lane; t < nkr * W; t += 64) krow[t] = 0.0;
+        wave_lds_sync();
+    }
     // K(row, col) += v: row = bra function fp + p (p < NP) or fq + q (NP + q); col the
     // molecule's function, ccol its LDS column
     auto kadd = [&](const int row, const int col, const int ccol, const double v) {
-        if (KROWS && row < nkr) {
+        if ((KROWS || WROWS) && row < nkr) {
             __hip_atomic_fetch_add(&krow[row * W + ccol], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         } else {
             unsafeAtomicAdd(&b.Y[(size_t)(row < NP ? fp + row : fq + row - NP) * ld + col], v);
@@ -745,9 +769,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
             // P is symmetric: P(s,q) etc. are read as P(q,s) from the bra pair's rows,
             // which every lane of the wavefront shares (cache-resident), instead of one
             // row per lane
-            // LDS columns of the ket's functions (KROWS)
+            // LDS columns of the ket's functions
             int ccr = 0, ccs = 0;
-            if (KROWS) {
+            if (KROWS || WROWS) {
                 const int kc = ldc(a.kcol + t.sk);
                 ccr = hi16(kc);
                 ccs = (LR == LS ? 0 : nR) + lo16(kc);
@@ -915,14 +939,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
         atomicAdd(&a.counters[3 * a.counter_slot + 1], npq);
         atomicAdd(&a.counters[3 * a.counter_slot + 2], n32);
     }
-    if (KROWS) {
-        // every wavefront of the work-group is here (one bra pair, no early return)
-        __syncthreads();
-        for (int t = threadIdx.x; t < nkr * W; t += blockDim.x) {
+    if (KROWS || WROWS) {
+        // KROWS: every wavefront of the work-group is here (one bra pair, no early return)
+        if (KROWS) __syncthreads();
+        else wave_lds_sync();
+        for (int t = KROWS ? (int)threadIdx.x : lane; t < nkr * W; t += KROWS ? (int)blockDim.x : 64) {
             const double v = krow[t];
             const int row = t / W, cc = t - row * W;
             if (v != 0.0) {
-                const int col = ldc(a.kcol_map + (cc < nR ? a.kcol_lofs[LR] + cc : a.kcol_lofs[LS] + cc - nR));
+                const int col = ldc(a.kcol_map + (cc < nR ? lofR + cc : lofS + cc - nR));
                 unsafeAtomicAdd(&b.Y[(size_t)(row < NP ? fp + row : fq + row - NP) * ld + col], v);
             }
         }

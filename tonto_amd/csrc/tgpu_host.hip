@@ -450,36 +450,25 @@ static const bool kHeavy[NQCLS] = {
 #undef TGPU_HEAVY_FLAG
 };
 
-// Default kernel form per class pair.  Single molecules: the lane-per-quartet form for
-// every class pair that has one but (fs|dp); with its K rows in LDS (columns of the ket
-// momenta only) it beat the wavefront form on those class pairs of (H2O)64 / cc-pVTZ
-// (tgpu_autotune, FP64 build at an SCF density: (pp|pp) 57 vs 125 ms, (ds|ds) 92 vs 377,
-// (fs|ps) 159 vs 400, (dp|ds) 218 vs 450, (dd|ps) 89 vs 230, (fp|ps) 120 vs 279, (dp|pp)
-// 124 vs 301, (fp|ds) 137 vs 207, (fd|ps) 122 vs 178; (fs|dp) 296 vs 215, its lane kernel
-// spilling 0.5-0.9 KB per lane).  Batches (no LDS rows): the wavefront form for the class
-// pairs whose lane kernels need more than 230 registers: (pp|pp), (ds|pp), (ds|ds),
-// (fs|ps), (fs|ds) and those with more than 81 integrals.  tgpu_autotune re-decides per
-// molecule.
-static bool wave_by_default_single(int lp, int lq, int lr, int ls)
+// Default kernel form per class pair: the lane-per-quartet form for every class pair that
+// has one, with these exceptions (class times of one build, lane against wavefront form):
+//   (ff|ss)               0.93 against 0.67 ms at (H2O)12/cc-pVTZ, 4.4 against 4.3 at (H2O)32
+//                         (its lane kernel updates K globally);
+//   (dp|pp) in batches    13.0 against 12.6 ms for 256 clusters in 6-31G(d,p), where
+//                         (ps|ps)-like classes are at 40 against 136 and (dd|ps) at 3.8
+//                         against 10.4;
+//   more than 100 integrals and few quartets (fewer than 2^19 bra-ket pairs of a single
+//   molecule): the lane kernels of these hold 400 to 512 registers, one wavefront per SIMD,
+//   and a small system does not fill the lanes: (dd|ps) 0.47 against 0.14 ms at
+//   (H2O)8/6-31G(d), (fp|ds) 1.02 against 0.48 at (H2O)5/cc-pVTZ, but (fp|ds) 1.3 against
+//   2.8 at (H2O)12/cc-pVTZ.
+// tgpu_autotune re-decides per context.
+static bool wave_by_default(int lp, int lq, int lr, int ls, bool batch, double quartets)
 {
-    return lp == 3 && lq == 0 && lr == 2 && ls == 1;
+    if (lp == 3 && lq == 3) return true;
+    if (batch) return lp == 2 && lq == 1 && lr == 1 && ls == 1;
+    return ncart(lp) * ncart(lq) * ncart(lr) * ncart(ls) > 100 && quartets < 524288.0;
 }
-static bool wave_by_default_batch(int lp, int lq, int lr, int ls)
-{
-    return (lp == 1 && lq == 1 && lr == 1 && ls == 1) || (lp == 2 && lq == 0 && lr == 1 && ls == 1) ||
-           (lp == 2 && lq == 0 && lr == 2 && ls == 0) || (lp == 3 && lq == 0 && lr == 1 && ls == 0) ||
-           (lp == 3 && lq == 0 && lr == 2 && ls == 0) || ncart(lp) * ncart(lq) * ncart(lr) * ncart(ls) > 81;
-}
-static const bool kWaveDefaultBatch[NQCLS] = {
-#define TGPU_WAVE_DEFAULT(LP, LQ, LR, LS, H) (H || wave_by_default_batch(LP, LQ, LR, LS)),
-    TGPU_FOR_EACH_CLASS(TGPU_WAVE_DEFAULT)
-#undef TGPU_WAVE_DEFAULT
-};
-static const bool kWaveDefaultSingle[NQCLS] = {
-#define TGPU_WAVE_DEFAULT(LP, LQ, LR, LS, H) (H || wave_by_default_single(LP, LQ, LR, LS)),
-    TGPU_FOR_EACH_CLASS(TGPU_WAVE_DEFAULT)
-#undef TGPU_WAVE_DEFAULT
-};
 
 // The class launches of a build are independent (every update is an atomic add), so they run
 // on the build's stream and kSide side streams, forked from it after the density maxima and
@@ -597,11 +586,13 @@ struct tgpu_ctx {
     std::vector<double> A, AB, maxI;
     std::vector<double> pz, pzi, pK, pPx, pPy, pPz;
     std::vector<int> bin_max_seg;  // [NBIN] largest molecule segment of each bin
-    // single molecule: number of each shell's first function among the functions of its
+    // per molecule: number of each shell's first function among the functions of its
     // angular momentum, and those functions grouped by momentum (the lane kernels' LDS
     // K rows hold only the columns of the ket shells' momenta)
     std::vector<int> sh_kcol, kcol_map;
-    int kcol_lofs[TGPU_LMAX + 2] = {0};
+    int kcol_lofs[TGPU_LMAX + 2] = {0};  // (single molecule)
+    std::vector<int> klofs;               // [n_mol * (TGPU_LMAX + 2)], positions in kcol_map
+    int kcol_max[TGPU_LMAX + 1] = {0};    // most functions of a momentum in a molecule
     bool have_schwarz = false;
     std::vector<double> maxI_mol, maxI_tonto;
     int variant[NQCLS];
@@ -609,7 +600,7 @@ struct tgpu_ctx {
     int chunk[NQCLS] = {0};
     // device
     DBuf<int> d_rec0, d_rec1, d_sh_l, d_sh_bf, d_seg_start, d_seg_count, d_nbf, d_shell_off,
-        d_atom_off, d_kcol, d_kcol_map;
+        d_atom_off, d_kcol, d_kcol_map, d_klofs;
     DBuf<long long> d_pair_off, d_mat_off;
     DBuf<double> d_A, d_AB, d_maxI, d_maxI_mol;
     DBuf<PrimRec> d_prim;
@@ -788,11 +779,14 @@ static int upload_pairs(tgpu_ctx *c)
     std::vector<PrimRec> prim(c->pz.size());
     for (size_t k = 0; k < prim.size(); ++k)
         prim[k] = PrimRec{c->pz[k], c->pzi[k], c->pK[k], c->pPx[k], c->pPy[k], c->pPz[k], 0.0, 0.0};
-    if (c->n_mol == 1) {
+    {
         // per pair: pack16(column number of its first shell's first function, of its
         // second shell's) within the functions of each shell's momentum
         std::vector<int> kc(c->tonto.size());
-        for (size_t k = 0; k < kc.size(); ++k) kc[k] = pack16(c->sh_kcol[c->sp[k]], c->sh_kcol[c->sq[k]]);
+        for (size_t k = 0; k < kc.size(); ++k) {
+            const int s0 = c->shell_off[c->pmol[k]];
+            kc[k] = pack16(c->sh_kcol[s0 + c->sp[k]], c->sh_kcol[s0 + c->sq[k]]);
+        }
         if ((rc = dupload(c, c->d_kcol, kc))) return rc;
     }
     if ((rc = dupload(c, c->d_rec0, r0)) || (rc = dupload(c, c->d_rec1, r1)) ||
@@ -1023,25 +1017,40 @@ extern "C" int tgpu_create_batch(const tgpu_system *sys, int n_mol, tgpu_ctx **o
             c->AB[3 * s + t] = c->xyz[3 * c->sh_atom[s0 + p] + t] - c->xyz[3 * c->sh_atom[s0 + q] + t];
         }
     }
-    if (n_mol == 1) {
-        // functions grouped by angular momentum, in shell order within each momentum
+    // functions grouped by molecule and angular momentum, in shell order within each momentum
+    c->sh_kcol.resize(c->sh_l.size());
+    c->klofs.assign((size_t)n_mol * (TGPU_LMAX + 2), 0);
+    for (int m = 0; m < n_mol; ++m) {
+        const int s0 = c->shell_off[m], s1 = c->shell_off[m + 1];
         int cnt[TGPU_LMAX + 1] = {0};
-        c->sh_kcol.resize(c->sh_l.size());
-        for (size_t sh = 0; sh < c->sh_l.size(); ++sh) {
+        for (int sh = s0; sh < s1; ++sh) {
             c->sh_kcol[sh] = cnt[c->sh_l[sh]];
             cnt[c->sh_l[sh]] += ncart(c->sh_l[sh]);
         }
-        c->kcol_lofs[0] = 0;
-        for (int l = 0; l <= TGPU_LMAX; ++l) c->kcol_lofs[l + 1] = c->kcol_lofs[l] + cnt[l];
-        c->kcol_map.assign(c->kcol_lofs[TGPU_LMAX + 1], 0);
-        for (size_t sh = 0; sh < c->sh_l.size(); ++sh)
+        int *lofs = &c->klofs[(size_t)m * (TGPU_LMAX + 2)];
+        lofs[0] = (int)c->kcol_map.size();
+        for (int l = 0; l <= TGPU_LMAX; ++l) {
+            lofs[l + 1] = lofs[l] + cnt[l];
+            c->kcol_max[l] = std::max(c->kcol_max[l], cnt[l]);
+        }
+        c->kcol_map.resize(lofs[TGPU_LMAX + 1], 0);
+        for (int sh = s0; sh < s1; ++sh)
             for (int k = 0; k < ncart(c->sh_l[sh]); ++k)
-                c->kcol_map[c->kcol_lofs[c->sh_l[sh]] + c->sh_kcol[sh] + k] = c->sh_bf[sh] + k;
+                c->kcol_map[lofs[c->sh_l[sh]] + c->sh_kcol[sh] + k] = c->sh_bf[sh] + k;
     }
+    if (n_mol == 1) std::copy(c->klofs.begin(), c->klofs.end(), c->kcol_lofs);
     build_prims(c);
-    for (int k = 0; k < NQCLS; ++k) c->variant[k] = (n_mol > 1 ? kWaveDefaultBatch[k] : kWaveDefaultSingle[k]) ? 1 : 0;
+    {
+        auto pairs = [&](int cls) { return (double)(c->bin_start[cls * NBK + NBK] - c->bin_start[cls * NBK]); };
+        int k = 0;
+#define TGPU_WAVE_DEFAULT(LP, LQ, LR, LS, H)                                                       \
+    c->variant[k++] = H || wave_by_default(LP, LQ, LR, LS, n_mol > 1,                              \
+                                           pairs(pair_class(LP, LQ)) * pairs(pair_class(LR, LS)));
+        TGPU_FOR_EACH_CLASS(TGPU_WAVE_DEFAULT)
+#undef TGPU_WAVE_DEFAULT
+    }
     int rc;
-    if (n_mol == 1 && (rc = dupload(c, c->d_kcol_map, c->kcol_map))) return rc;
+    if ((rc = dupload(c, c->d_kcol_map, c->kcol_map)) || (rc = dupload(c, c->d_klofs, c->klofs))) return rc;
     if ((rc = upload_pairs(c))) return rc;
     if ((rc = dupload(c, c->d_sh_l, c->sh_l)) || (rc = dupload(c, c->d_sh_bf, c->sh_bf)) ||
         (rc = dupload(c, c->d_nbf, c->nbf)) || (rc = dupload(c, c->d_shell_off, c->shell_off)) ||
@@ -1087,7 +1096,7 @@ extern "C" int tgpu_destroy(tgpu_ctx *c)
     dfree(c->d_rec0); dfree(c->d_rec1); dfree(c->d_sh_l); dfree(c->d_sh_bf);
     dfree(c->d_seg_start); dfree(c->d_seg_count); dfree(c->d_nbf); dfree(c->d_shell_off);
     dfree(c->d_atom_off); dfree(c->d_pair_off); dfree(c->d_mat_off);
-    dfree(c->d_kcol); dfree(c->d_kcol_map);
+    dfree(c->d_kcol); dfree(c->d_kcol_map); dfree(c->d_klofs);
     dfree(c->d_A); dfree(c->d_AB); dfree(c->d_maxI); dfree(c->d_maxI_mol); dfree(c->d_prim);
     dfree(c->d_X); dfree(c->d_Y);
     dfree(c->d_bin_start); dfree(c->d_bin_boff); dfree(c->d_PP); dfree(c->d_XP);
@@ -1449,8 +1458,11 @@ static int enqueue_build(tgpu_ctx *c, const BuildBufs &B, const double *P, doubl
     a.prow_enable = c->prow_enable;
     a.n_shell = c->n_mol == 1 ? (int)c->sh_l.size() : 0;
     a.pmrow = c->pmrow_enable;
-    a.kcol = c->n_mol == 1 ? c->d_kcol.p : nullptr;
-    a.kcol_map = c->n_mol == 1 ? c->d_kcol_map.p : nullptr;
+    a.kcol = c->d_kcol.p;
+    a.kcol_map = c->d_kcol_map.p;
+    a.klofs = c->d_klofs.p;
+    for (int l = 0; l <= TGPU_LMAX; ++l) a.kcol_max[l] = c->kcol_max[l];
+    a.krow_stride = 0;
     for (int l = 0; l <= TGPU_LMAX + 1; ++l) a.kcol_lofs[l] = c->kcol_lofs[l];
     const bool prof = rec_end && c->profiling;
     // one stream where each class pair is timed, and where the caller is capturing s
