@@ -390,7 +390,8 @@ struct JKArgs {
     // accumulator copies (single molecules): X and Y hold TGPU_ACC_COPIES copies acc_stride
     // doubles apart and a wavefront adds into the copy of the XCD it runs on (0: one copy)
     long long acc_stride;
-    unsigned long long *counters;
+    unsigned long long *counters;  // [counter_copies][TGPU_COUNTER_STRIDE]
+    int counter_copies;            // a power of two
 };
 
 // One launch covers every bin pair of a class pair that runs in the same kernel form: work-
@@ -441,6 +442,25 @@ __device__ __forceinline__ int take_part(const JKLaunch &L, JKArgs &a, int &gx, 
 // by one XCD only.  Any copy index gives the same sums (the atomics stay device-scope),
 // so the index only has to be in range.
 #define TGPU_ACC_COPIES 8
+
+// Copies of the class counters.  Atomics on one address take their turn at 14 ns each, three
+// per wavefront: with one copy every class of 256 clusters took 45 ns per wavefront, whatever
+// it computed ((ps|ss): 2.0e6 wavefronts, 94 ms).  A work-group adds to the copy of its index.
+#ifndef TGPU_COUNTER_COPIES
+#define TGPU_COUNTER_COPIES 16
+#endif
+// one copy: 3 per class pair, whole cache lines
+constexpr int TGPU_COUNTER_STRIDE = (3 * TGPU_NPAIRCLASS * (TGPU_NPAIRCLASS + 1) / 2 + 15) / 16 * 16;
+
+__device__ __forceinline__ void count_quartets(const JKArgs &a, unsigned long long nq, unsigned long long npq,
+                                               unsigned long long n32)
+{
+    unsigned long long *const c =
+        a.counters + (blockIdx.x & (a.counter_copies - 1)) * TGPU_COUNTER_STRIDE + 3 * a.counter_slot;
+    atomicAdd(c, nq);
+    if (npq) atomicAdd(c + 1, npq);
+    if (n32) atomicAdd(c + 2, n32);
+}
 
 // The XCD the wavefront runs on (hardware register XCC_ID), reduced to a copy index.
 __device__ __forceinline__ int acc_copy()
@@ -934,11 +954,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
         npq += __shfl_xor(npq, off, 64);
         n32 += __shfl_xor(n32, off, 64);
     }
-    if (lane == 0 && nq) {
-        atomicAdd(&a.counters[3 * a.counter_slot + 0], nq);
-        atomicAdd(&a.counters[3 * a.counter_slot + 1], npq);
-        atomicAdd(&a.counters[3 * a.counter_slot + 2], n32);
-    }
+    if (lane == 0 && nq) count_quartets(a, nq, npq, n32);
     if (KROWS || WROWS) {
         // KROWS: every wavefront of the work-group is here (one bra pair, no early return)
         if (KROWS) __syncthreads();
@@ -1418,9 +1434,7 @@ __device__ void wave_bra(const JKArgs &a, int bi, int y, int gy, WaveLDS<LP, LQ,
         npq += __shfl_xor(npq, off, 64);
     }
     if (lane == 0 && nq) {
-        atomicAdd(&a.counters[3 * a.counter_slot + 0], nq);
-        atomicAdd(&a.counters[3 * a.counter_slot + 1], npq);
-        if (F32) atomicAdd(&a.counters[3 * a.counter_slot + 2], nq);
+        count_quartets(a, nq, npq, F32 ? nq : 0);
     }
     wave_lds_sync();  // LDS is reused by the work-group's next bra pair
 }
@@ -1942,9 +1956,7 @@ __device__ void wave_bra(const JKArgs &a, int bi, int y, int gy, WaveLDS<LP, LQ,
         npq += __shfl_xor(npq, off, 64);
     }
     if (lane == 0 && nq) {
-        atomicAdd(&a.counters[3 * a.counter_slot + 0], nq);
-        atomicAdd(&a.counters[3 * a.counter_slot + 1], npq);
-        if (F32) atomicAdd(&a.counters[3 * a.counter_slot + 2], nq);
+        count_quartets(a, nq, npq, F32 ? nq : 0);
     }
     __syncthreads();  // L is reused by the work-group's next bra pair
 }

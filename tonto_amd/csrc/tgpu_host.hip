@@ -1075,7 +1075,7 @@ extern "C" int tgpu_create_batch(const tgpu_system *sys, int n_mol, tgpu_ctx **o
     if ((rc = dalloc(c, c->d_X, (size_t)c->n_elem * c->acc_copies)) ||
         (rc = dalloc(c, c->d_Y, (size_t)c->n_elem * c->acc_copies)) ||
         (rc = dalloc(c, c->d_Pmax, (size_t)c->n_pairs)) || (rc = dalloc(c, c->d_scal, 2 * (size_t)n_mol)) ||
-        (rc = dalloc(c, c->d_maxI_mol, (size_t)n_mol)) || (rc = dalloc(c, c->d_counters, 3 * NQCLS)))
+        (rc = dalloc(c, c->d_maxI_mol, (size_t)n_mol)) || (rc = dalloc(c, c->d_counters, TGPU_COUNTER_COPIES * TGPU_COUNTER_STRIDE)))
         return rc;
     HIPCHK(c, hipEventCreate(&c->ev0));
     HIPCHK(c, hipEventCreate(&c->ev1));
@@ -1309,20 +1309,21 @@ static int grid_for(size_t n) { return (int)std::min<size_t>((n + 255) / 256, 16
 
 // Device buffers one build writes besides J and K: the accumulators X, Y (n_elem doubles
 // each), P_max per Tonto pair, the per-molecule maxima (2 per molecule), the class counters
-// (3 per class pair) and the wavefront-form workspace.
+// (3 per class pair, in counter_copies copies) and the wavefront-form workspace.
 struct BuildBufs {
     double *X, *Y, *Pmax, *scal;
     unsigned long long *counters;
     double *ws;
     long long ws_doubles;
     int acc_copies;  // copies of X and Y (n_elem doubles apart)
+    int counter_copies;
     double *PP, *XP;  // pair-ordered ket blocks (bin_boff[NBIN] doubles each)
 };
 
 static BuildBufs ctx_bufs(const tgpu_ctx *c)
 {
     return BuildBufs{c->d_X.p,       c->d_Y.p,    c->d_Pmax.p,      c->d_scal.p,  c->d_counters.p,
-                     c->d_ws.p,      c->ws_doubles, c->acc_copies, c->d_PP.p, c->d_XP.p};
+                     c->d_ws.p,      c->ws_doubles, c->acc_copies, TGPU_COUNTER_COPIES, c->d_PP.p, c->d_XP.p};
 }
 
 // Largest per-slot workspace (doubles) of the wavefront-form class pairs this basis has
@@ -1415,7 +1416,8 @@ static int enqueue_build(tgpu_ctx *c, const BuildBufs &B, const double *P, doubl
     const long long n_acc = c->n_elem * B.acc_copies;
     fill_zero_kernel<<<grid_for(n_acc), 256, 0, s>>>(B.X, n_acc);
     fill_zero_kernel<<<grid_for(n_acc), 256, 0, s>>>(B.Y, n_acc);
-    fill_zero_u64_kernel<<<(3 * NQCLS + 255) / 256, 256, 0, s>>>(B.counters, 3 * NQCLS);
+    const int n_cnt = B.counter_copies * TGPU_COUNTER_STRIDE;
+    fill_zero_u64_kernel<<<(n_cnt + 255) / 256, 256, 0, s>>>(B.counters, n_cnt);
     // the pair-ordered ket blocks: each pair's density block in, the ket-side J out
     const PairBlocks pbk{c->d_bin_start.p, c->d_bin_boff.p, reinterpret_cast<const int4 *>(c->d_rec0.p),
                          reinterpret_cast<const int4 *>(c->d_rec1.p), c->d_mat_off.p, c->d_nbf.p, c->n_pairs_dev()};
@@ -1448,6 +1450,7 @@ static int enqueue_build(tgpu_ctx *c, const BuildBufs &B, const double *P, doubl
     a.XP = B.XP;
     a.acc_stride = B.acc_copies > 1 ? c->n_elem : 0;
     a.counters = B.counters;
+    a.counter_copies = B.counter_copies;
     a.ws = B.ws;
     a.ws_doubles = B.ws_doubles;
     a.max_nbf = *std::max_element(c->nbf.begin(), c->nbf.end());
@@ -1623,10 +1626,10 @@ extern "C" int tgpu_make_r_JK_device(tgpu_ctx *c, const double *P, double *J, do
 }
 
 __global__ void copy_u64_kernel(unsigned long long *__restrict__ dst, const unsigned long long *__restrict__ src,
-                                int n)
+                                int n_src, int n_dst)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = src[i];
+    if (i < n_dst) dst[i] = i < n_src ? src[i] : 0ull;
 }
 
 // The build of tgpu_make_r_JK_device with every buffer it writes besides J and K carved
@@ -1680,23 +1683,30 @@ extern "C" int tgpu_make_r_JK_device_noalloc(tgpu_ctx *c, const double *P, doubl
         c->err = "tgpu_make_r_JK_device_noalloc: no scratch address for this device";
         return TGPU_E_STATE;
     }
+    // as many copies of the counters as fit
+    const size_t b_cnt1 = TGPU_COUNTER_STRIDE * sizeof(unsigned long long);
+    int copies = TGPU_COUNTER_COPIES;
+    while (copies > 1 && fixed + ws_slot + up(copies * b_cnt1) - b_cnt > TGPU_NOALLOC_SCRATCH_BYTES) copies /= 2;
     BuildBufs B;
     size_t off = 0;
     B.X = reinterpret_cast<double *>(base + off); off += b_mat;
     B.Y = reinterpret_cast<double *>(base + off); off += b_mat;
     B.Pmax = reinterpret_cast<double *>(base + off); off += b_pmax;
     B.scal = reinterpret_cast<double *>(base + off); off += b_scal;
-    B.counters = reinterpret_cast<unsigned long long *>(base + off); off += b_cnt;
+    B.counters = reinterpret_cast<unsigned long long *>(base + off); off += copies > 1 ? up(copies * b_cnt1) : b_cnt;
     B.PP = reinterpret_cast<double *>(base + off); off += b_blk;
     B.XP = reinterpret_cast<double *>(base + off); off += b_blk;
     B.ws = ws_slot ? reinterpret_cast<double *>(base + off) : nullptr;
     B.ws_doubles = ws_slot ? (long long)((TGPU_NOALLOC_SCRATCH_BYTES - off) / sizeof(double)) : 0;
     B.acc_copies = 1;
+    B.counter_copies = copies;
     const int kflags = flags & (TGPU_JK_MIXED | TGPU_J_ONLY | TGPU_K_ONLY);
     const SideLease side(c->device, false);  // (a new set would be an allocation)
     if (int rc = enqueue_build(c, B, P, J, K, kflags, c->stream, side.set, true, true)) return rc;
     // the context's own counters take this build's, so tgpu_get_stats reports it
-    copy_u64_kernel<<<1, 256, 0, c->stream>>>(c->d_counters.p, B.counters, 3 * NQCLS);
+    const int n_cnt = TGPU_COUNTER_COPIES * TGPU_COUNTER_STRIDE;
+    copy_u64_kernel<<<(n_cnt + 255) / 256, 256, 0, c->stream>>>(c->d_counters.p, B.counters, copies * TGPU_COUNTER_STRIDE,
+                                                             n_cnt);
     c->timed = true;
     HIPCHK(c, hipGetLastError());
     return TGPU_OK;
@@ -1785,14 +1795,24 @@ extern "C" int tgpu_make_r_JK(tgpu_ctx *c, const double *P, double *J, double *K
     return TGPU_OK;
 }
 
+// The class counters of the last build, summed over their copies.
+static int read_counters(tgpu_ctx *c, unsigned long long *out)
+{
+    std::vector<unsigned long long> h(TGPU_COUNTER_COPIES * TGPU_COUNTER_STRIDE);
+    HIPCHK(c, hipMemcpy(h.data(), c->d_counters.p, h.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost));
+    std::fill(out, out + 3 * NQCLS, 0ull);
+    for (int k = 0; k < TGPU_COUNTER_COPIES; ++k)
+        for (int i = 0; i < 3 * NQCLS; ++i) out[i] += h[k * TGPU_COUNTER_STRIDE + i];
+    return TGPU_OK;
+}
+
 extern "C" int tgpu_get_stats(tgpu_ctx *c, tgpu_stats *st)
 {
     if (!c || !st) return TGPU_E_ARG;
     std::memset(st, 0, sizeof(*st));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     std::vector<unsigned long long> h(3 * NQCLS);
-    HIPCHK(c, hipMemcpy(h.data(), c->d_counters.p, h.size() * sizeof(unsigned long long),
-                        hipMemcpyDeviceToHost));
+    if (int rc = read_counters(c, h.data())) return rc;
     for (int k = 0; k < NQCLS; ++k) {
         st->quartets += h[3 * k];
         st->prim_quartets += h[3 * k + 1];
@@ -1810,9 +1830,7 @@ extern "C" int tgpu_get_class_counters(tgpu_ctx *c, unsigned long long *out, int
 {
     if (!c || !out || n < 3 * NQCLS) return TGPU_E_ARG;
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    HIPCHK(c, hipMemcpy(out, c->d_counters.p, 3 * NQCLS * sizeof(unsigned long long),
-                        hipMemcpyDeviceToHost));
-    return TGPU_OK;
+    return read_counters(c, out);
 }
 
 extern "C" int tgpu_n_class_pairs(void) { return NQCLS; }
