@@ -282,17 +282,13 @@ def gen_wave(LP, LQ, LR, LS):
            f"    static constexpr int NP = {NP}, NQ = {NQ}, NR = {NR}, NS = {NS}, NROOT = {nroot};",
            f"    static constexpr int LPQ = {LPQ}, LRS = {LRS}, NE = {NE}, NF = {NF}, BUF = {buf};",
            f"    static constexpr int NCD = {len(cd)}, NAB = {len(ab)};",
-           arr("gidx", gidx),
+           arr("gidx", [gidx[3 * k] | gidx[3 * k + 1] << 6 | gidx[3 * k + 2] << 12 for k in range(len(gidx) // 3)], "int"),
            arr("cd_n", [len(l) for l in cd] or [0], "int"),
            arr("cd_off", [sum(len(x) for x in cd[:i]) for i in range(len(cd))] or [0], "int"),
-           arr("cd_s1", [e[0] for l in cd for e in l]),
-           arr("cd_s2", [e[1] for l in cd for e in l]),
-           arr("cd_ax", [e[2] for l in cd for e in l], "char"),
+           arr("cd_t", [e[0] | e[1] << 15 | e[2] << 30 for l in cd for e in l], "unsigned"),
            arr("ab_n", [len(l) for l in ab] or [0], "int"),
            arr("ab_off", [sum(len(x) for x in ab[:i]) for i in range(len(ab))] or [0], "int"),
-           arr("ab_s1", [e[0] for l in ab for e in l]),
-           arr("ab_s2", [e[1] for l in ab for e in l]),
-           arr("ab_ax", [e[2] for l in ab for e in l], "char"),
+           arr("ab_t", [e[0] | e[1] << 15 | e[2] << 30 for l in ab for e in l], "unsigned"),
            "};"]
     return "\n".join(out)
 

@@ -3,6 +3,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <utility>
+
 #include "../../include/tonto_gpu.h"
 #include "gen/classes.inc"
 #include "gen/sph.inc"
@@ -1607,6 +1609,75 @@ __device__ __forceinline__ WaveBuf<LP, LQ, LR, LS, R> &wave_buf(WaveLDS<LP, LQ, 
     else return L.u.f;
 }
 
+// Entries a lane has under way in the loops over LDS or workspace entries: one entry's chain
+// of latencies (table, two sources, result) after another bounded them, with 1 to 2 wavefronts
+// per SIMD.  Index tables are one word per entry and the level sizes compile-time.
+// (H2O)32/cc-pVTZ mixed, sum of the f classes' launches: 383 ms one at a time, 327 with 4, 289
+// with 6 (and the shift vector in registers), 291 with 8, where (ff|ps) goes from 6.5 to 11.5;
+// workspace classes, further from their data: 62.8 with 6, 60.9 with 8.
+__host__ __device__ constexpr int wave_unroll(int total, int lanes, int most)
+{
+    const int it = (total + lanes - 1) / lanes, rounds = (it + most - 1) / most;
+    return (it + rounds - 1) / rounds;  // no more than `most`, and the rounds even
+}
+
+template <typename R>
+struct Shift {
+    R x, y, z;
+};
+
+// One transfer level: dst[i] = src[base(i) + s1] + D[ax] src[base(i) + s2] for TOT entries,
+// the table word of entry i holding s1 | s2 << 15 | ax << 30.
+template <int TOT, int S, int MOST, typename R, typename Word, typename Index>
+__device__ __forceinline__ void transfer_level(const R *src, R *dst, const Shift<R> D, int tl, Word &&word, Index &&index)
+{
+    constexpr int U = wave_unroll(TOT, S, MOST);
+    for (int i0 = tl; i0 < TOT; i0 += U * S) {
+        unsigned w[U];
+        R v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) w[u] = word(min(i0 + u * S, TOT - 1));
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = min(i0 + u * S, TOT - 1);
+            const unsigned ax = w[u] >> 30;
+            v[u] = src[index(i, w[u] & 0x7fff)] + (ax == 0 ? D.x : ax == 1 ? D.y : D.z) * src[index(i, w[u] >> 15 & 0x7fff)];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (i0 + u * S < TOT) dst[i0 + u * S] = v[u];
+    }
+    __syncthreads();
+}
+
+template <typename T, int S, int MOST, int LEV, typename R>
+__device__ __forceinline__ void ket_level(const R *src, R *dst, const Shift<R> D, int tl)
+{
+    constexpr int n = T::cd_n[LEV], off = T::cd_off[LEV], nprev = LEV ? T::cd_n[LEV ? LEV - 1 : 0] : T::NF;
+    transfer_level<T::NE * n, S, MOST>(src, dst, D, tl, [](int i) { return T::cd_t[off + i % n]; },
+                                 [](int i, int s) { return i / n * nprev + s; });
+}
+
+template <typename T, int S, int MOST, int LEV, typename R>
+__device__ __forceinline__ void bra_level(const R *src, R *dst, const Shift<R> D, int tl)
+{
+    constexpr int n = T::ab_n[LEV], off = T::ab_off[LEV], NRS = T::NR * T::NS;
+    transfer_level<n * NRS, S, MOST>(src, dst, D, tl, [](int i) { return T::ab_t[off + i / NRS]; },
+                               [](int i, int s) { return s * NRS + i % NRS; });
+}
+
+template <typename T, int S, int MOST, typename R, int... LEV>
+__device__ __forceinline__ void ket_levels(R *b0, R *b1, const Shift<R> D, int tl, std::integer_sequence<int, LEV...>)
+{
+    (ket_level<T, S, MOST, LEV>(LEV % 2 ? b1 : b0, LEV % 2 ? b0 : b1, D, tl), ...);
+}
+
+template <typename T, int S, int MOST, typename R, int... LEV>
+__device__ __forceinline__ void bra_levels(R *b0, R *b1, const Shift<R> D, int tl, std::integer_sequence<int, LEV...>)
+{
+    (bra_level<T, S, MOST, LEV>(LEV % 2 ? b1 : b0, LEV % 2 ? b0 : b1, D, tl), ...);
+}
+
 // Computes (pq|rs) of one contracted quartet per team; returns the team's buffer holding
 // [pq][rs] (LDS, or the work-group's workspace slot gbuf of 2*BUF values for the classes
 // that keep their transfer buffers in global memory).  R is the type of the 2-D tables,
@@ -1643,14 +1714,13 @@ __device__ const R *wave_eri(const DevPrims &pm, const PairView &bra, const Pair
             Gr[m] = (R)0;
             const int k = tl + S * m;
             const int kk = k < NG ? k : 0;
-            gi[m] = T::gidx[3 * kk] | (T::gidx[3 * kk + 1] << 6) | (T::gidx[3 * kk + 2] << 12);
+            gi[m] = T::gidx[kk];
         }
-    } else {
-        // each lane owns entries tl, tl+S, ... until the transfer step
-        for (int k = tl; k < NG; k += S) src[k] = (R)0;
     }
     const int ax = tl / N, rr = tl - (tl / N) * N;
     const int np = live ? bra.n * ket.n : 0;
+    if (!C::GREG && np == 0)
+        for (int k = tl; k < NG; k += S) src[k] = (R)0;
     for (int ipq = 0; ipq < npmax; ++ipq) {
         const bool on = ipq < np;
         if (on && tl < 3 * N) {
@@ -1705,13 +1775,28 @@ __device__ const R *wave_eri(const DevPrims &pm, const PairView &bra, const Pair
                     Gr[m] += acc;
                 }
             } else {
-                for (int k = tl; k < NG; k += S) {
-                    const int i0 = T::gidx[3 * k], i1 = TW * N + T::gidx[3 * k + 1],
-                              i2 = 2 * TW * N + T::gidx[3 * k + 2];
-                    R acc = (R)0;
+                // each lane owns entries tl, tl + S, ... until the transfer step
+                constexpr int U = wave_unroll(NG, S, C::GB ? 4 : 6);
+                for (int k0 = tl; k0 < NG; k0 += U * S) {
+                    int g[U];
+                    R v[U];
 #pragma unroll
-                    for (int r = 0; r < N; ++r) acc += B.g[i0 + r * TW] * B.g[i1 + r * TW] * B.g[i2 + r * TW];
-                    src[k] += acc;
+                    for (int u = 0; u < U; ++u) {
+                        const int k = min(k0 + u * S, NG - 1);
+                        g[u] = T::gidx[k];
+                        v[u] = ipq ? src[k] : (R)0;
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const int i0 = g[u] & 63, i1 = TW * N + ((g[u] >> 6) & 63), i2 = 2 * TW * N + (g[u] >> 12);
+                        R acc = (R)0;
+#pragma unroll
+                        for (int r = 0; r < N; ++r) acc += B.g[i0 + r * TW] * B.g[i1 + r * TW] * B.g[i2 + r * TW];
+                        v[u] += acc;
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        if (k0 + u * S < NG) src[k0 + u * S] = v[u];
                 }
             }
         }
@@ -1725,31 +1810,14 @@ __device__ const R *wave_eri(const DevPrims &pm, const PairView &bra, const Pair
         }
     }
     __syncthreads();
-    // ket-side transfer, rows e (T::NE of them), entries per level
-    const R CD[3] = {(R)ket.ABx, (R)ket.ABy, (R)ket.ABz};
-    int nprev = T::NF;
-    for (int lev = 0; lev < T::NCD; ++lev) {
-        const int n = T::cd_n[lev], off = T::cd_off[lev];
-        for (int idx = tl; idx < T::NE * n; idx += S) {
-            const int e = idx / n, t = idx - e * n;
-            dst[e * n + t] = src[e * nprev + T::cd_s1[off + t]] + CD[T::cd_ax[off + t]] * src[e * nprev + T::cd_s2[off + t]];
-        }
-        __syncthreads();
-        R *tmp = src; src = dst; dst = tmp;
-        nprev = n;
-    }
-    // bra-side transfer on columns rs
-    const R AB[3] = {(R)bra.ABx, (R)bra.ABy, (R)bra.ABz};
-    for (int lev = 0; lev < T::NAB; ++lev) {
-        const int n = T::ab_n[lev], off = T::ab_off[lev];
-        for (int idx = tl; idx < n * NRS; idx += S) {
-            const int t = idx / NRS, c = idx - t * NRS;
-            dst[t * NRS + c] = src[T::ab_s1[off + t] * NRS + c] + AB[T::ab_ax[off + t]] * src[T::ab_s2[off + t] * NRS + c];
-        }
-        __syncthreads();
-        R *tmp = src; src = dst; dst = tmp;
-    }
-    return src;
+    // ket-side transfer on rows e, then bra-side on columns rs; the result ends in buffer
+    // (NCD + NAB) % 2
+    const Shift<R> CD{(R)ket.ABx, (R)ket.ABy, (R)ket.ABz};
+    ket_levels<T, S, C::GB ? 8 : 6>(src, dst, CD, tl, std::make_integer_sequence<int, T::NCD>());
+    const Shift<R> AB{(R)bra.ABx, (R)bra.ABy, (R)bra.ABz};
+    if constexpr (T::NCD % 2 == 0) bra_levels<T, S, C::GB ? 8 : 6>(src, dst, AB, tl, std::make_integer_sequence<int, T::NAB>());
+    else bra_levels<T, S, C::GB ? 8 : 6>(dst, src, AB, tl, std::make_integer_sequence<int, T::NAB>());
+    return (T::NCD + T::NAB) % 2 == 0 ? src : dst;
 }
 
 
@@ -1964,11 +2032,15 @@ __device__ void wave_bra(const JKArgs &a, int bi, int y, int gy, WaveLDS<LP, LQ,
 // Wavefront form: a part's grid is (gx, gy); its work-group (x, y), number y * gx + x, takes
 // bra pairs x, x + gx, ... and, of each, the ket chunks y, y + gy, ...  Workspace classes keep
 // the launch's work-groups <= their slot count and use the work-group's number as slot.
-#ifndef TGPU_WAVE_MIN_WAVES
-#define TGPU_WAVE_MIN_WAVES 1
-#endif
+// Wavefronts per SIMD the registers are kept to: three in the class pairs that lost their
+// third to the loops above and gain from it ((H2O)32/cc-pVTZ mixed: (fp|dp) 25.2 -> 21.7 ms,
+// (fs|dd) 10.1 -> 8.9; any other class pair is slower or the same)
+__host__ __device__ constexpr int wave_min_waves(int lp, int lq, int lr, int ls)
+{
+    return (lp == 3 && lq == 1 && lr == 2 && ls == 1) || (lp == 3 && lq == 0 && lr == 2 && ls == 2) ? 3 : 1;
+}
 template <int LP, int LQ, int LR, int LS, typename R>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(TGPU_WAVE_MIN_WAVES, 8))) void jk_wave_kernel(JKLaunch J)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(wave_min_waves(LP, LQ, LR, LS), 8))) void jk_wave_kernel(JKLaunch J)
 {
     JKArgs a = J.a;
     int gx, gy;
