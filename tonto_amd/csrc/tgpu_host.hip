@@ -322,13 +322,18 @@ struct OneEArgs {
     double *S, *T, *V;
 };
 
+// kOneELanes neighbouring lanes share a pair's nuclei: with one lane per pair the launches waited
+// for a few long chains over all nuclei ((H2O)16/cc-pVTZ, 48 nuclei: the whole call 6.5 ms with 1
+// lane, 3.2 with 16).
+constexpr int kOneELanes = 16;
+
 // pairs: (first shell, second shell, molecule) with l(first) = LA, l(second) = LB
 template <int LA, int LB>
 __global__ __launch_bounds__(64) void one_e_kernel(OneEArgs a, const int4 *__restrict__ pairs, int n)
 {
     constexpr int NA = ncart(LA), NB = ncart(LB), L = LA + LB, NR = L / 2 + 1;
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= n) return;
+    const int g = (int)(blockIdx.x * 64 + threadIdx.x) / kOneELanes, sub = threadIdx.x & (kOneELanes - 1);
+    if (g >= n) return;  // uniform over a pair's lanes
     const int4 pr = pairs[g];
     const int x = pr.x, y = pr.y, m = pr.z;
     const int nbf = a.b.nbf[m];
@@ -358,6 +363,7 @@ __global__ __launch_bounds__(64) void one_e_kernel(OneEArgs a, const int4 *__res
             for (int i = 0; i < NA; ++i)
 #pragma unroll
                 for (int j = 0; j < NB; ++j) {
+                    if (sub) continue;
                     double s3[3], t3[3];
 #pragma unroll
                     for (int t = 0; t < 3; ++t) {
@@ -371,7 +377,7 @@ __global__ __launch_bounds__(64) void one_e_kernel(OneEArgs a, const int4 *__res
                     sb[i][j] += pre * s3[0] * s3[1] * s3[2];
                     tb[i][j] += pre * (t3[0] * s3[1] * s3[2] + s3[0] * t3[1] * s3[2] + s3[0] * s3[1] * t3[2]);
                 }
-            for (int C = a.b.atom_off[m]; C < a.b.atom_off[m + 1]; ++C) {
+            for (int C = a.b.atom_off[m] + sub; C < a.b.atom_off[m + 1]; C += kOneELanes) {
                 const double *Cc = a.xyz + 3 * C;
                 double PC2 = 0.0;
                 for (int t = 0; t < 3; ++t) PC2 += (Pc[t] - Cc[t]) * (Pc[t] - Cc[t]);
@@ -410,6 +416,13 @@ __global__ __launch_bounds__(64) void one_e_kernel(OneEArgs a, const int4 *__res
                 }
             }
         }
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int off = kOneELanes / 2; off > 0; off >>= 1) vb[i][j] += __shfl_xor(vb[i][j], off, 64);
+    if (sub) return;
     const int fa = a.b.sh_bf[x], fb = a.b.sh_bf[y];
 #pragma unroll
     for (int i = 0; i < NA; ++i)
@@ -2004,7 +2017,7 @@ extern "C" int tgpu_one_electron(tgpu_ctx *c, double *S, double *T, double *V)
     {                                                                                         \
         const int k = pair_class(LP, LQ);                                                     \
         const int n = (int)(cls_start[k + 1] - cls_start[k]);                                 \
-        if (n) one_e_kernel<LP, LQ><<<(n + 63) / 64, 64, 0, c->stream>>>(a, d_pairs.p + cls_start[k], n); \
+        if (n) one_e_kernel<LP, LQ><<<(unsigned)((kOneELanes * (long long)n + 63) / 64), 64, 0, c->stream>>>(a, d_pairs.p + cls_start[k], n); \
     }
     TGPU_FOR_EACH_PAIRCLASS(TGPU_ONE_E_CASE)
 #undef TGPU_ONE_E_CASE
