@@ -708,61 +708,80 @@ static void drop_graph(tgpu_ctx *c)
 // (shell1quartet.foo:201-270) so that the skip decisions are bit-identical.
 static void build_prims(tgpu_ctx *c)
 {
-    c->pz.clear(); c->pzi.clear(); c->pK.clear(); c->pPx.clear(); c->pPy.clear(); c->pPz.clear();
     const size_t np = c->tonto.size();
     c->off_full.assign(np, 0); c->n_full.assign(np, 0);
     c->off_skip.assign(np, 0); c->n_skip.assign(np, 0);
     // all full runs in pair order, then all skipped runs: neighbouring lanes of a
     // wavefront (neighbouring ket pairs) then read neighbouring primitive records
-    for (int pass = 0; pass < 2; ++pass) {
-        const bool skip = pass == 1;
-        for (size_t s = 0; s < np; ++s) {
-            const int m = c->pmol[s], s0 = c->shell_off[m];
-            const int ab = c->tonto[s];
-            int a = (int)((std::sqrt(8.0 * ab + 1.0) - 1.0) / 2.0);
-            while (a * (a + 1) / 2 > ab) --a;
-            while ((a + 1) * (a + 2) / 2 <= ab) ++a;
-            const int b = ab - a * (a + 1) / 2 + s0;
-            a += s0;
-            const double *PA = &c->xyz[3 * c->sh_atom[a]], *PB = &c->xyz[3 * c->sh_atom[b]];
-            const bool same = c->sh_atom[a] == c->sh_atom[b];
-            if (skip && same) {  // never used: a quartet with a same-atom pair keeps full lists
-                c->off_skip[s] = c->off_full[s];
-                c->n_skip[s] = c->n_full[s];
-                continue;
-            }
-            const double ABv[3] = {PA[0] - PB[0], PA[1] - PB[1], PA[2] - PB[2]};
-            const double r2 = ABv[0] * ABv[0] + ABv[1] * ABv[1] + ABv[2] * ABv[2];
-            const int off = (int)c->pz.size();
-            for (int bg = 0; bg < c->sh_np[b]; ++bg) {
-                const double be = c->exps[c->sh_off[b] + bg], bcc = c->coefs[c->sh_off[b] + bg];
-                const double b_r2 = be * r2;
-                for (int ag = 0; ag < c->sh_np[a]; ++ag) {
-                    const double ae = c->exps[c->sh_off[a] + ag], acc = c->coefs[c->sh_off[a] + ag];
-                    const double sum = ae + be, inv = 1.0 / sum;
-                    const double cc = bcc * acc * inv * std::sqrt(inv);
-                    double pref, P[3];
-                    if (same) {
-                        pref = cc;
-                        P[0] = PA[0]; P[1] = PA[1]; P[2] = PA[2];
-                    } else {
-                        const double e = std::exp(-ae * b_r2 * inv);
-                        if (skip && e < c->cut_pair) continue;
-                        pref = cc * e;
-                        for (int t = 0; t < 3; ++t) P[t] = (be * PB[t] + ae * PA[t]) * inv;
-                    }
-                    c->pz.push_back(sum);
-                    c->pzi.push_back(inv);
-                    c->pK.push_back(pref);
-                    c->pPx.push_back(P[0]);
-                    c->pPy.push_back(P[1]);
-                    c->pPz.push_back(P[2]);
+    std::vector<int> sa(np), sb(np);
+    size_t total = 0;
+    for (size_t s = 0; s < np; ++s) {
+        const int s0 = c->shell_off[c->pmol[s]];
+        const int ab = c->tonto[s];
+        int a = (int)((std::sqrt(8.0 * ab + 1.0) - 1.0) / 2.0);
+        while (a * (a + 1) / 2 > ab) --a;
+        while ((a + 1) * (a + 2) / 2 <= ab) ++a;
+        sb[s] = ab - a * (a + 1) / 2 + s0;
+        sa[s] = a + s0;
+        c->off_full[s] = (int)total;
+        c->n_full[s] = c->sh_np[sa[s]] * c->sh_np[sb[s]];
+        total += c->n_full[s];
+    }
+    std::vector<double> *const cols[6] = {&c->pz, &c->pzi, &c->pK, &c->pPx, &c->pPy, &c->pPz};
+    for (auto *v : cols) v->resize(total);
+    // the skipped runs are the full runs' primitives with an exponential factor of at least
+    // cut_pair, taken from there: the exponentials are most of the work
+    std::vector<char> keep(total);
+    size_t n_keep = 0;
+    for (size_t s = 0; s < np; ++s) {
+        const int a = sa[s], b = sb[s];
+        const double *PA = &c->xyz[3 * c->sh_atom[a]], *PB = &c->xyz[3 * c->sh_atom[b]];
+        const bool same = c->sh_atom[a] == c->sh_atom[b];
+        const double ABv[3] = {PA[0] - PB[0], PA[1] - PB[1], PA[2] - PB[2]};
+        const double r2 = ABv[0] * ABv[0] + ABv[1] * ABv[1] + ABv[2] * ABv[2];
+        size_t i = c->off_full[s];
+        for (int bg = 0; bg < c->sh_np[b]; ++bg) {
+            const double be = c->exps[c->sh_off[b] + bg], bcc = c->coefs[c->sh_off[b] + bg];
+            const double b_r2 = be * r2;
+            for (int ag = 0; ag < c->sh_np[a]; ++ag, ++i) {
+                const double ae = c->exps[c->sh_off[a] + ag], acc = c->coefs[c->sh_off[a] + ag];
+                const double sum = ae + be, inv = 1.0 / sum;
+                const double cc = bcc * acc * inv * std::sqrt(inv);
+                double pref, P[3];
+                if (same) {
+                    pref = cc;
+                    P[0] = PA[0]; P[1] = PA[1]; P[2] = PA[2];
+                } else {
+                    const double e = std::exp(-ae * b_r2 * inv);
+                    keep[i] = !(e < c->cut_pair);
+                    n_keep += keep[i];
+                    pref = cc * e;
+                    for (int t = 0; t < 3; ++t) P[t] = (be * PB[t] + ae * PA[t]) * inv;
                 }
+                c->pz[i] = sum;
+                c->pzi[i] = inv;
+                c->pK[i] = pref;
+                c->pPx[i] = P[0];
+                c->pPy[i] = P[1];
+                c->pPz[i] = P[2];
             }
-            const int n = (int)c->pz.size() - off;
-            if (!skip) { c->off_full[s] = off; c->n_full[s] = n; }
-            else { c->off_skip[s] = off; c->n_skip[s] = n; }
         }
+    }
+    for (auto *v : cols) v->resize(total + n_keep);
+    size_t off = total;
+    for (size_t s = 0; s < np; ++s) {
+        if (c->sh_atom[sa[s]] == c->sh_atom[sb[s]]) {  // never used: a quartet with a same-atom pair keeps full lists
+            c->off_skip[s] = c->off_full[s];
+            c->n_skip[s] = c->n_full[s];
+            continue;
+        }
+        c->off_skip[s] = (int)off;
+        for (size_t i = c->off_full[s], end = i + c->n_full[s]; i < end; ++i)
+            if (keep[i]) {
+                for (auto *v : cols) (*v)[off] = (*v)[i];
+                ++off;
+            }
+        c->n_skip[s] = (int)off - c->off_skip[s];
     }
 }
 
