@@ -48,10 +48,10 @@ SCHWARZ, FP32_THR = 1e-11, 1e-6
 # WRITE_SIZE passes scaled by what the same counters read for a 256 MiB copy (x2.000 and
 # x1.000): the profiles/ traffic summary of (H2O)64 / cc-pVTZ
 TRAFFIC = {
-    "jk class (21|21) mixed": {"bytes": 2.512824e+11, "read": 1.807234e+11, "written": 7.055901e+10, "dispatches": 6},
-    "jk class (20|10) mixed": {"bytes": 9.951025e+11, "read": 8.881830e+11, "written": 1.069195e+11, "dispatches": 12},
-    "jk class (10|00) mixed": {"bytes": 5.139057e+11, "read": 4.466742e+11, "written": 6.723149e+10, "dispatches": 16},
-    "jk class (10|10) mixed": {"bytes": 1.251133e+12, "read": 1.139521e+12, "written": 1.116115e+11, "dispatches": 10},
+    "jk class (21|21) mixed": {"bytes": 1.555449e+11, "read": 1.090239e+11, "written": 4.652096e+10, "dispatches": 2},
+    "jk class (20|10) mixed": {"bytes": 6.888888e+11, "read": 6.150393e+11, "written": 7.384945e+10, "dispatches": 1},
+    "jk class (10|00) mixed": {"bytes": 3.156562e+11, "read": 2.935462e+11, "written": 2.210996e+10, "dispatches": 1},
+    "jk class (10|10) mixed": {"bytes": 8.188299e+11, "read": 7.449846e+11, "written": 7.384534e+10, "dispatches": 1},
 }
 
 
