@@ -1,4 +1,4 @@
-"""The network's kernel forms at the sizes where they can go wrong, against the numpy checker:
+"""The network's kernel forms at the sizes where they can go wrong, against the numpy reference:
 row blocks and tiles with remainders, a batch longer than one work-group's share of the
 weight gradients, a net whose row block exceeds the LDS (general products).  FP32 sums of K
 terms in another order: |error| <= 2^-24 (2 K)^(1/2) 8 max|result| with K the longest sum,
@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n_in,nh,n_out,M", [(1, 1, 1, 1), (273, 128, 225, 2047), (33, 31, 17, 16), (64, 48, 32, 17),
                                              (1000, 300, 900, 50), (9, 8, 5, 33000), (700, 16, 3, 200)])
-def test_forms_against_checker(n_in, nh, n_out, M):
+def test_forms_against_reference(n_in, nh, n_out, M):
     import torch
     if not torch.cuda.is_available():
         pytest.fail("no HIP device visible: GPU tests must run on an MI355X")
