@@ -36,7 +36,7 @@ def class_list():
 
 
 def _deps(extra):
-    return [os.path.join(CSRC, f) for f in ("tgpu_device.h", "rys_table.inc")] + \
+    return [os.path.join(CSRC, f) for f in ("tgpu_device.h", "launch_plan.h", "rys_table.inc")] + \
         [os.path.join(CSRC, "gen", "classes.inc"), os.path.join(CSRC, "gen", "pair_form.inc"), os.path.join(HERE, "..", "include", "tonto_gpu.h")] + extra
 
 

@@ -4,6 +4,7 @@
 #include <algorithm>
 
 #include "tgpu_device.h"
+#include "launch_plan.h"
 
 #define TGPU_STR2(x) #x
 #define TGPU_STR(x) TGPU_STR2(x)
@@ -145,11 +146,6 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, cons
     constexpr bool kGB = C::GB;  // transfer buffers in the workspace
     constexpr long long kWS = C::WS;
 #endif
-    // work-group (x, y) of a part: bra pairs x, x + gx, ...; of each, ket chunks y, y + gy,
-    // ... of ket_chunk kets.  gy splits long prefixes when there are few bra pairs, so that
-    // a part's grid holds about kWaveGrid work-groups; the launches of workspace classes
-    // stay within their slots, shared evenly by the parts.
-    constexpr long long kWaveGrid = 65536;
     JKLaunch L;
     L.a = a;
     L.n_part = n_part;
@@ -168,25 +164,22 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, cons
                     return rc;
             return TGPU_OK;
         }
-        slots /= n_part;
     }
-    long long grid = 0;
+    WavePlan plan[TGPU_MAX_PARTS];
     for (int k = 0; k < n_part; ++k) {
         JKPart &p = L.part[k];
         p = parts[k];
         if (p.ket_chunk <= 0 || p.ket_chunk > 64) p.ket_chunk = 64;  // one lane per ket
-        const long long nch = p.n_ket_max > 0 ? (p.n_ket_max + p.ket_chunk - 1) / p.ket_chunk : 1;
-        long long gx = p.n_bra, gy;
-        if (kGB) {
-            gx = std::min<long long>(gx, slots);
-            gy = std::min<long long>(nch, std::max<long long>(1, slots / gx));
-        } else {
-            gy = std::min<long long>(nch, std::max<long long>(1, (kWaveGrid + gx - 1) / gx));
-        }
-        p.gx = (int)gx;
-        p.gy = (int)gy;
+        plan[k] = WavePlan{p.n_bra, p.n_ket_max > 0 ? (p.n_ket_max + p.ket_chunk - 1) / p.ket_chunk : 1, 0, 0};
+    }
+    plan_wave(plan, n_part, slots);
+    long long grid = 0;
+    for (int k = 0; k < n_part; ++k) {
+        JKPart &p = L.part[k];
+        p.gx = (int)plan[k].gx;
+        p.gy = (int)plan[k].gy;
         p.first = (int)grid;
-        grid += gx * gy;
+        grid += plan[k].gx * plan[k].gy;
     }
     if (grid > 0x3ffffffLL) return TGPU_E_UNSUPPORTED;  // fewer than 2^32 threads
     jk_wave_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, double><<<(unsigned)grid, 64, 0, s>>>(L);
