@@ -666,6 +666,46 @@ struct tgpu_ctx {
         }                                                                              \
     } while (0)
 
+// The workspace of a destroyed context, kept for the next one on its device.  The driver wipes
+// freed memory at about 35 GB/s, and allocations wait for that once a program frees faster:
+// set-ups of (H2O)5/cc-pVTZ in a loop, each with 1 GiB allocated and freed, took 24 to 30 ms
+// (95th percentile 145 to 175, longest 3.2 s), 3.1 ms (3.2, 4.3) with the workspace sized and
+// kept.  One buffer per device, at most kWsMost (0.4 % of the card's memory), freed when an
+// allocation of this library fails.  A buffer is put here only when the work on it is
+// done (after a hipFree, which waits for the device).
+constexpr size_t kWsMost = (size_t)1 << 30;  // bytes
+struct WsPool {
+    static std::mutex mu;
+    static DBuf<double> kept[kMaxDevices];
+
+    // the kept buffer if it holds n doubles, else none
+    static DBuf<double> take(int device, size_t n)
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        DBuf<double> b;
+        if (kept[device].p && kept[device].n >= n) std::swap(b, kept[device]);
+        return b;
+    }
+    static void put(int device, DBuf<double> &b)
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        if (b.p && b.n > kept[device].n && b.n * sizeof(double) <= kWsMost) std::swap(b, kept[device]);
+        if (b.p) (void)hipFree(b.p);
+        b = DBuf<double>();
+    }
+    // frees the kept buffer; false if there was none
+    static bool release(int device)
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        const bool had = kept[device].p;
+        if (had) (void)hipFree(kept[device].p);
+        kept[device] = DBuf<double>();
+        return had;
+    }
+};
+std::mutex WsPool::mu;
+DBuf<double> WsPool::kept[kMaxDevices];
+
 template <typename T>
 static int dalloc(tgpu_ctx *c, DBuf<T> &b, size_t n)
 {
@@ -674,7 +714,13 @@ static int dalloc(tgpu_ctx *c, DBuf<T> &b, size_t n)
     b.p = nullptr;
     b.n = 0;
     if (n == 0) n = 1;
-    HIPCHK(c, hipMalloc((void **)&b.p, n * sizeof(T)));
+    hipError_t e = hipMalloc((void **)&b.p, n * sizeof(T));
+    if (e == hipErrorOutOfMemory && WsPool::release(c->device)) {
+        (void)hipGetLastError();
+        e = hipMalloc((void **)&b.p, n * sizeof(T));
+    }
+    if (e != hipSuccess) b.p = nullptr;
+    HIPCHK(c, e);
     b.n = n;
     return 0;
 }
@@ -1135,7 +1181,7 @@ extern "C" int tgpu_destroy(tgpu_ctx *c)
     dfree(c->d_Pmax); dfree(c->d_scal); dfree(c->d_hP); dfree(c->d_hJ); dfree(c->d_hK);
     dfree(c->d_hP2); dfree(c->d_hJ2); dfree(c->d_hK2); dfree(c->d_uJ); dfree(c->d_uK);
     dfree(c->d_counters);
-    dfree(c->d_ws);
+    WsPool::put(c->device, c->d_ws);  // (the hipFree before waited for the work on it)
     dfree(c->d_sh_sbf); dfree(c->d_cbf_shell); dfree(c->d_sbf_shell);
     dfree(c->d_Pc); dfree(c->d_Jc); dfree(c->d_Kc);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -1259,15 +1305,34 @@ static const int kClassPair[NQCLS][2] = {
 #undef TGPU_CLASSPAIR
 };
 
-// Allocates the wavefront-form workspace for the class pairs this basis has (none for
-// s/p/d bases): room for at least 1024 slots of the largest per-slot need, and up to
-// 8192 slots or 1 GiB, so classes with smaller transfer buffers run wider grids.
-static size_t workspace_need(const tgpu_ctx *c);
+// The wavefront-form workspace of the class pairs that keep their transfer buffers there (none
+// for s/p/d bases): the slots that the widest of their launches can use (a bra pair and a
+// chunk of at least 16 kets each, at most 8192), up to kWsMost.  One water in cc-pVTZ needs
+// 0.3 MB, five 48 MB, twelve 560 MB; (H2O)64 takes 2937 ms with 1 GiB, 3015 with 512 MiB.
+static size_t workspace_wanted(const tgpu_ctx *c)
+{
+    size_t most = 0;
+    for (int k = 0; k < NQCLS; ++k) {
+        const int CX = kClassPair[k][0], CY = kClassPair[k][1];
+        const size_t ws = kWaveWs[k]();
+        if (!ws) continue;
+        long long slots = 0;
+        for (int bx = 0; bx < NBK; ++bx)
+            for (int by = 0; by < (CX == CY ? bx + 1 : NBK); ++by) {
+                const int X = CX * NBK + bx, Y = CY * NBK + by;
+                const long long chunks = (c->bin_max_seg[Y] + 15) / 16;
+                slots += chunks * (c->bin_start[X + 1] - c->bin_start[X]);
+            }
+        most = std::max(most, ws * (size_t)std::min(slots, 8192LL));
+    }
+    return std::min(most, kWsMost / sizeof(double));
+}
+
 static int ensure_workspace(tgpu_ctx *c)
 {
-    const size_t need = workspace_need(c);
-    if (!need) return 0;
-    const size_t n = std::max(1024 * need, std::min(8192 * need, (size_t)(1 << 30) / sizeof(double)));
+    const size_t n = workspace_wanted(c);
+    if (!n || (c->d_ws.p && c->d_ws.n >= n)) return 0;
+    if (!c->d_ws.p) c->d_ws = WsPool::take(c->device, n);
     if (int rc = dalloc(c, c->d_ws, n)) return rc;
     c->ws_doubles = (long long)n;
     return 0;
