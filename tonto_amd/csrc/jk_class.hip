@@ -3,8 +3,8 @@
 // -DTGPU_LS=.. -DTGPU_HEAVY=0|1.
 #include <algorithm>
 
-#include "tgpu_device.h"
 #include "launch_plan.h"
+#include "tgpu_device.h"
 
 #define TGPU_STR2(x) #x
 #define TGPU_STR(x) TGPU_STR2(x)
@@ -22,15 +22,14 @@
 int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, const JKPart *parts, int n_part,
                                                          int variant, bool mixed, hipStream_t s)
 {
-    if (n_part <= 0 || n_part > TGPU_MAX_PARTS) return TGPU_OK;
+    if (n_part <= 0) return TGPU_OK;
+    if (n_part > TGPU_MAX_PARTS) return TGPU_E_ARG;
 #if !TGPU_HEAVY
     if (variant == 0) {
         // parts in the LDS-row form, then the others four bra pairs per work-group
         JKLaunch rows, glob;
         rows.a = glob.a = a;
-        rows.n_part = glob.n_part = 0;
-        int rows_grid = 0, glob_grid = 0;
-        size_t lds = 0;
+        size_t lds = 0, wlds = 0;
         // The LDS-row form for single molecules with long ket segments (>= 4 rounds of 64 by
         // default, so that the four wavefronts of one bra pair have work): as many of the
         // bra pair's K rows as fit the work-group's LDS budget next to the Rys table and
@@ -87,50 +86,58 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, cons
                           : 0;
             if (b.pmrow) lds += pm_bytes;
         }
+        // The others: the rows of the wavefronts' own bra pairs in LDS, at most kWaveRowsLds per
+        // work-group if all of them then fit (two work-groups per CU), else as many as fit one,
+        // down to a quarter of them; global updates only for (ff|ss) (as above), where K is not
+        // digested, and for molecules too large for a quarter.
+        constexpr size_t kWaveRowsLds = 76 * 1024;
+        const size_t Wmax = a.kcol_max[TGPU_LR] + (TGPU_LR == TGPU_LS ? 0 : a.kcol_max[TGPU_LS]);
+        const size_t row4 = 4 * Wmax * sizeof(double);  // one row of each wavefront
+        const size_t room = budget > kStatic ? budget - kStatic : 0;
+        const size_t small = budget < kWaveRowsLds ? room : kWaveRowsLds - kStatic;
+        int nwr = row4 ? (int)std::min<size_t>(NP + NQ, small / row4) : 0;
+        if (nwr < NP + NQ && row4) nwr = (int)std::min<size_t>(NP + NQ, room / row4);
+        if (a.kp != HUGE_VAL && a.kcol && 4 * nwr >= NP + NQ) {
+            glob.a.krow_rows = nwr;
+            glob.a.krow_stride = (int)(nwr * Wmax);
+            wlds = nwr * row4;
+        }
 #endif
+        auto in_rows = [&](const JKPart &p) { return rows_ok && p.n_ket_avg >= a.krow_min_kets; };
+        long long groups[TGPU_MAX_PARTS];
         for (int k = 0; k < n_part; ++k) {
-            const bool r = rows_ok && parts[k].n_ket_avg >= a.krow_min_kets;
-            JKLaunch &L = r ? rows : glob;
-            JKPart &p = L.part[L.n_part++];
-            p = parts[k];
-            p.gx = p.gy = 1;
-            p.first = r ? rows_grid : glob_grid;
-            if (r) rows_grid += p.n_bra;
-            else glob_grid += (p.n_bra + 3) / 4;
+            groups[k] = in_rows(parts[k]) ? parts[k].n_bra : (parts[k].n_bra + 3LL) / 4;
+            if (groups[k] > kMostThreads / 256) return TGPU_E_UNSUPPORTED;
         }
-#if !(TGPU_LP == 3 && TGPU_LQ == 3 && TGPU_LR == 0 && TGPU_LS == 0)
-        if (rows_grid > 0) {
-            if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, KR_GROUP><<<rows_grid, 256, lds, s>>>(rows);
-            else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, KR_GROUP><<<rows_grid, 256, lds, s>>>(rows);
-        }
-#endif
-        if (glob_grid > 0) {
-            // The rows of the wavefronts' own bra pairs in LDS, at most kWaveRowsLds per work-
-            // group if all of them then fit (two work-groups per CU), else as many as fit one,
-            // down to a quarter of them; global updates only for (ff|ss) (as above), where K is
-            // not digested, and for molecules too large for a quarter.
-            size_t wlds = 0;
-#if !(TGPU_LP == 3 && TGPU_LQ == 3 && TGPU_LR == 0 && TGPU_LS == 0)
-            constexpr size_t kWaveRowsLds = 76 * 1024;
-            const size_t Wmax = a.kcol_max[TGPU_LR] + (TGPU_LR == TGPU_LS ? 0 : a.kcol_max[TGPU_LS]);
-            const size_t row4 = 4 * Wmax * sizeof(double);  // one row of each wavefront
-            const size_t room = budget > kStatic ? budget - kStatic : 0;
-            const size_t small = budget < kWaveRowsLds ? room : kWaveRowsLds - kStatic;
-            int nwr = row4 ? (int)std::min<size_t>(NP + NQ, small / row4) : 0;
-            if (nwr < NP + NQ && row4) nwr = (int)std::min<size_t>(NP + NQ, room / row4);
-            if (a.kp != HUGE_VAL && a.kcol && 4 * nwr >= NP + NQ) {
-                glob.a.krow_rows = nwr;
-                glob.a.krow_stride = (int)(nwr * Wmax);
-                wlds = nwr * row4;
+        for (int k0 = 0, k1; k0 < n_part; k0 = k1) {
+            k1 = launch_end(groups, n_part, k0, kMostThreads / 256);
+            int rows_grid = 0, glob_grid = 0;
+            rows.n_part = glob.n_part = 0;
+            for (int k = k0; k < k1; ++k) {
+                const bool r = in_rows(parts[k]);
+                JKLaunch &L = r ? rows : glob;
+                JKPart &p = L.part[L.n_part++];
+                p = parts[k];
+                p.gx = p.gy = 1;
+                int &grid = r ? rows_grid : glob_grid;
+                p.first = grid;
+                grid += (int)groups[k];
             }
-            if (wlds) {
+#if !(TGPU_LP == 3 && TGPU_LQ == 3 && TGPU_LR == 0 && TGPU_LS == 0)
+            if (rows_grid > 0) {
+                if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, KR_GROUP><<<rows_grid, 256, lds, s>>>(rows);
+                else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, KR_GROUP><<<rows_grid, 256, lds, s>>>(rows);
+            }
+            if (glob_grid > 0 && wlds) {
                 if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, KR_WAVE><<<glob_grid, 256, wlds, s>>>(glob);
                 else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, KR_WAVE><<<glob_grid, 256, wlds, s>>>(glob);
-                return TGPU_OK;
+                continue;
             }
 #endif
-            if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, KR_GLOBAL><<<glob_grid, 256, 0, s>>>(glob);
-            else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, KR_GLOBAL><<<glob_grid, 256, 0, s>>>(glob);
+            if (glob_grid > 0) {
+                if (mixed) jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, true, KR_GLOBAL><<<glob_grid, 256, 0, s>>>(glob);
+                else jk_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, false, KR_GLOBAL><<<glob_grid, 256, 0, s>>>(glob);
+            }
         }
         return TGPU_OK;
     }
@@ -148,7 +155,6 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, cons
 #endif
     JKLaunch L;
     L.a = a;
-    L.n_part = n_part;
     // FP64 over the kets before the FP32 split of each prefix (all of it in an FP64 build),
     // then FP32 over the rest
     if (!mixed) L.a.fp32_thr = 0.0;
@@ -166,24 +172,33 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, cons
         }
     }
     WavePlan plan[TGPU_MAX_PARTS];
+    long long groups[TGPU_MAX_PARTS];
+    auto chunk = [](const JKPart &p) { return p.ket_chunk > 0 && p.ket_chunk <= 64 ? p.ket_chunk : 64; };  // one lane per ket
     for (int k = 0; k < n_part; ++k) {
-        JKPart &p = L.part[k];
-        p = parts[k];
-        if (p.ket_chunk <= 0 || p.ket_chunk > 64) p.ket_chunk = 64;  // one lane per ket
-        plan[k] = WavePlan{p.n_bra, p.n_ket_max > 0 ? (p.n_ket_max + p.ket_chunk - 1) / p.ket_chunk : 1, 0, 0};
+        const int nk = parts[k].n_ket_max, kc = chunk(parts[k]);
+        plan[k] = WavePlan{parts[k].n_bra, nk > 0 ? (nk + kc - 1) / kc : 1, 0, 0};
     }
     plan_wave(plan, n_part, slots);
-    long long grid = 0;
     for (int k = 0; k < n_part; ++k) {
-        JKPart &p = L.part[k];
-        p.gx = (int)plan[k].gx;
-        p.gy = (int)plan[k].gy;
-        p.first = (int)grid;
-        grid += plan[k].gx * plan[k].gy;
+        groups[k] = plan[k].gx * plan[k].gy;
+        if (groups[k] > kMostThreads / 64) return TGPU_E_UNSUPPORTED;
     }
-    if (grid > 0x3ffffffLL) return TGPU_E_UNSUPPORTED;  // fewer than 2^32 threads
-    jk_wave_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, double><<<(unsigned)grid, 64, 0, s>>>(L);
-    if (mixed) jk_wave_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, float><<<(unsigned)grid, 64, 0, s>>>(L);
+    for (int k0 = 0, k1; k0 < n_part; k0 = k1) {
+        k1 = launch_end(groups, n_part, k0, kMostThreads / 64);
+        int grid = 0;
+        L.n_part = k1 - k0;
+        for (int k = k0; k < k1; ++k) {
+            JKPart &p = L.part[k - k0];
+            p = parts[k];
+            p.ket_chunk = chunk(p);
+            p.gx = (int)plan[k].gx;
+            p.gy = (int)plan[k].gy;
+            p.first = grid;
+            grid += (int)groups[k];
+        }
+        jk_wave_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, double><<<grid, 64, 0, s>>>(L);
+        if (mixed) jk_wave_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, float><<<grid, 64, 0, s>>>(L);
+    }
     return TGPU_OK;
 }
 
@@ -215,7 +230,11 @@ void TGPU_SCHWARZ_NAME_X(TGPU_LP, TGPU_LQ)(const DevPairs &pr, const DevPrims &p
     (void)ws;
     (void)ws_doubles;
     constexpr int kSplit = 16;
-    schwarz_kernel<TGPU_LP, TGPU_LQ, kSplit><<<(n + 64 / kSplit - 1) / (64 / kSplit), 64, 0, s>>>(pr, pm, start, n, maxI, sph);
+    // (the lanes are numbered in an int)
+    in_chunks(n, (1LL << 31) / kSplit, [&](long long at, long long count) {
+        const int grid = (int)((count + 64 / kSplit - 1) / (64 / kSplit));
+        schwarz_kernel<TGPU_LP, TGPU_LQ, kSplit><<<grid, 64, 0, s>>>(pr, pm, start + (int)at, (int)count, maxI, sph);
+    });
 #endif
 }
 #endif

@@ -39,3 +39,24 @@ inline void plan_wave(WavePlan *p, int n, long long slots)
         p[k].gy = gy;
     }
 }
+
+// A launch has to have fewer than 2^32 threads along x.
+constexpr long long kMostThreads = 0xffffffffLL;
+
+// The bin pairs [first, end) go into one launch of at most `most` work-groups; a bin pair that
+// has more by itself is alone.  (A class pair's 16 bin pairs together can exceed the limit that
+// each keeps to: (ps|ss) from about 4.2 million bra pairs.)
+inline int launch_end(const long long *groups, int n, int first, long long most)
+{
+    long long sum = groups[first];
+    int end = first + 1;
+    while (end < n && sum + groups[end] <= most) sum += groups[end++];
+    return end;
+}
+
+// f(at, count) for consecutive parts of n items, at most `most` each
+template <typename F>
+inline void in_chunks(long long n, long long most, F f)
+{
+    for (long long at = 0; at < n; at += most) f(at, std::min(most, n - at));
+}

@@ -28,6 +28,7 @@
 #include <string>
 #include <vector>
 
+#include "launch_plan.h"
 #include "tgpu_device.h"
 
 static constexpr int NCLS = TGPU_NPAIRCLASS;
@@ -2100,8 +2101,11 @@ extern "C" int tgpu_one_electron(tgpu_ctx *c, double *S, double *T, double *V)
 #define TGPU_ONE_E_CASE(LP, LQ, H)                                                              \
     {                                                                                         \
         const int k = pair_class(LP, LQ);                                                     \
-        const int n = (int)(cls_start[k + 1] - cls_start[k]);                                 \
-        if (n) one_e_kernel<LP, LQ><<<(unsigned)((kOneELanes * (long long)n + 63) / 64), 64, 0, c->stream>>>(a, d_pairs.p + cls_start[k], n); \
+        const int4 *const pr = d_pairs.p + cls_start[k];                                      \
+        in_chunks(cls_start[k + 1] - cls_start[k], (1LL << 31) / kOneELanes, [&](long long at, long long n) { \
+            const int grid = (int)((kOneELanes * n + 63) / 64);                               \
+            one_e_kernel<LP, LQ><<<grid, 64, 0, c->stream>>>(a, pr + at, (int)n);             \
+        });                                                                                   \
     }
     TGPU_FOR_EACH_PAIRCLASS(TGPU_ONE_E_CASE)
 #undef TGPU_ONE_E_CASE
