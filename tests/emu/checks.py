@@ -6,7 +6,10 @@ import sys
 
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__)))))
 
-from tonto_amd.gpu import lib  # noqa: E402
+import numpy as np  # noqa: E402
+
+from tonto_amd.geometry import water_cluster  # noqa: E402
+from tonto_amd.gpu import JKEngine, TGPUError, lib  # noqa: E402
 
 
 class Emu:
@@ -24,6 +27,9 @@ class Emu:
             name = self.L.emu_entry(i, v).decode()
             out.append((name,) + tuple(v))
         return out
+
+    def fail(self, name, n):
+        self.L.emu_fail(name.encode(), n)
 
     def launches(self):
         """(kernel, stream, threads, grid x, grid y, block, LDS bytes) of every launch"""
@@ -71,6 +77,128 @@ def launch_limits():
     ls = e.launches()
     assert all(threads < 2 ** 32 for _, _, threads, *_ in ls), ls
     assert sum(4 * l[3] for l in ls) >= n
+
+
+def _density(n, seed):
+    A = np.random.default_rng(seed).standard_normal((n, n))
+    return 0.5 * A @ A.T / n
+
+
+class Build:
+    """A context with its matrices (device memory is host memory here)."""
+
+    def __init__(self, mol, seed=0, **options):
+        self.mol, self.eng = mol, JKEngine(mol, **options)
+        self.max_I = self.eng.schwarz()
+        self.P = _density(self.eng.n_bf, seed)
+        self.J, self.K = np.empty_like(self.P), np.empty_like(self.P)
+
+    def run(self, **flags):
+        self.J.fill(np.nan)
+        self.K.fill(np.nan)
+        self.eng.make_r_JK_device(self.P.ctypes.data, self.J.ctypes.data, self.K.ctypes.data, **flags)
+        return self.J.copy(), self.K.copy()
+
+
+def failing_runtime_calls():
+    """A fork, join, launch or capture that fails ends the build with an error, forked streams are
+    joined all the same, and the next build is right."""
+    e = Emu()
+    b = Build(water_cluster(1, "STO-3G", seed=1))
+    J0, K0 = b.run()
+
+    def fails(name, n, what, **flags):
+        e.L.emu_clear()
+        e.fail(name, n)
+        try:
+            b.run(**flags)
+        except TGPUError:
+            pass
+        else:
+            raise AssertionError(f"{what} failed and the build went on")
+        finally:
+            e.fail("", -1)
+        failed = e.log()
+        b.eng.set_cutoffs_scaled(1.0)  # (a captured build runs at its capture only)
+        J, K = b.run(**flags)
+        assert abs(J - J0).max() < 1e-14 and abs(K - K0).max() < 1e-14, what
+        return failed
+    for flags in (dict(), dict(graph=True)):
+        if flags:
+            b.eng.set_cutoffs_scaled(1.0)  # (drops the captured build)
+        e.L.emu_clear()
+        b.run(**flags)
+        log = e.log()
+        waited = {x[2] for x in log if x[0] == "hipStreamWaitEvent"}
+        records = [x for x in log if x[0] == "hipEventRecord"]
+        n_fork = len([x for x in log if x[0] == "hipStreamWaitEvent"])
+        n_launch = len(e.launches())
+        assert n_fork >= 6 and len(records) >= 4 and n_launch > 6, (n_fork, records, n_launch)
+        for n, r in enumerate(records):
+            if r[2] in waited and n in (0, 1, 2, len(records) - 1, len(records) - 2):  # (the others are timing events)
+                b.eng.set_cutoffs_scaled(1.0)
+                fails("hipEventRecord", n, f"record {n} of {flags}", **flags)
+        for n in sorted({0, 1, 2, n_fork // 2, n_fork - 1}):
+            b.eng.set_cutoffs_scaled(1.0)
+            log = fails("hipStreamWaitEvent", n, f"wait {n} of {flags}", **flags)
+            # no launch on a side stream without a join or a host wait after it, unless captured
+            if not flags:
+                done = {x[1] for x in log if x[0] in ("hipEventRecord", "hipStreamSynchronize")}
+                assert {l[1] for l in log if l[5] > 0} <= done | {0}, log
+        for n in (0, 8, n_launch - 1):
+            b.eng.set_cutoffs_scaled(1.0)
+            fails("launch", n, f"launch {n} of {flags}", **flags)
+    # a failed capture: its side streams go, and no later build uses them
+    b.eng.set_cutoffs_scaled(1.0)
+    log = fails("hipStreamEndCapture", 0, "the capture", graph=True)
+    gone = {x[1] for x in log if x[0] == "hipStreamDestroy"}
+    assert len(gone) == 3, log
+    assert gone.isdisjoint({l[1] for l in e.launches()[len(log):]})
+    # no side streams to be had: the build runs in series
+    e.fail("hipStreamCreate", 0)
+    b2 = Build(water_cluster(1, "STO-3G", seed=1))
+    e.fail("", -1)
+    J, K = b2.run()
+    assert abs(J - J0).max() < 1e-14 and abs(K - K0).max() < 1e-14
+
+
+def kept_workspace():
+    """A destroyed context leaves its workspace to the next; an allocation that fails frees it and
+    is tried again."""
+    e = Emu()
+    mol = water_cluster(1, "cc-pVTZ", seed=1)
+    first = JKEngine(mol)
+    first.schwarz()
+    first.close()
+    e.L.emu_clear()
+    second = JKEngine(mol)
+    second.schwarz()
+    with_kept = len([x for x in e.log() if x[0] == "hipMalloc"])
+    third = JKEngine(mol)
+    e.L.emu_clear()
+    third.schwarz()
+    alone = len([x for x in e.log() if x[0] == "hipMalloc"])
+    second.close()  # (leaves the larger workspace or the same)
+    e.L.emu_clear()
+    fourth = JKEngine(mol)
+    n_create = len([x for x in e.log() if x[0] == "hipMalloc"])
+    fourth.schwarz()
+    assert with_kept - n_create == alone - 1, (with_kept, n_create, alone)
+    fourth.close()
+    e.fail("hipMalloc", 0)
+    fifth = JKEngine(mol)  # the kept buffer makes room
+    e.fail("hipMalloc", 0)
+    try:
+        JKEngine(mol)  # nothing is kept now
+    except TGPUError:
+        pass
+    else:
+        raise AssertionError("no error")
+    e.fail("", -1)
+    e.L.emu_clear_error()
+    fifth.schwarz()
+    third.close()
+    fifth.close()
 
 
 if __name__ == "__main__":

@@ -202,6 +202,7 @@ void emu_fail(const char *name, int n)
     emu::fail_after = n;
 }
 void emu_clear() { emu::log.clear(); }
+void emu_clear_error() { emu::last = hipSuccess; }
 int emu_size() { return (int)emu::log.size(); }
 const char *emu_entry(int i, long long *v)
 {

@@ -29,3 +29,11 @@ def emulated(tmp_path_factory):
 
 def test_launch_limits(emulated):
     emulated("launch_limits")
+
+
+def test_failing_runtime_calls(emulated):
+    emulated("failing_runtime_calls")
+
+
+def test_kept_workspace(emulated):
+    emulated("kept_workspace")

@@ -537,6 +537,7 @@ struct SidePool {
         SideSet *p = new SideSet();
         if (!p->make()) {
             delete p;
+            (void)hipGetLastError();  // the build goes on without
             return nullptr;
         }
         ++made[device];
@@ -547,6 +548,13 @@ struct SidePool {
         if (!p) return;
         std::lock_guard<std::mutex> lock(mu);
         idle[device].push_back(p);
+    }
+    static void discard(int device, SideSet *p)
+    {
+        if (!p) return;
+        std::lock_guard<std::mutex> lock(mu);
+        delete p;
+        --made[device];
     }
     static void add_ctx(int device)
     {
@@ -571,9 +579,14 @@ int SidePool::made[kMaxDevices], SidePool::n_ctx[kMaxDevices];
 // A set held by one call
 struct SideLease {
     const int device;
-    SideSet *const set;
+    SideSet *set;
     SideLease(int d, bool create) : device(d), set(SidePool::get(d, create)) {}
     ~SideLease() { SidePool::put(device, set); }
+    void discard()
+    {
+        SidePool::discard(device, set);
+        set = nullptr;
+    }
     SideLease(const SideLease &) = delete;
     SideLease &operator=(const SideLease &) = delete;
 };
@@ -1575,16 +1588,27 @@ static int enqueue_build(tgpu_ctx *c, const BuildBufs &B, const double *P, doubl
     int on[NQCLS];
     std::vector<int> order;
     assign_streams(c, fork, on, order);
+    // A failed fork would let a class kernel run before the accumulators are cleared, a failed
+    // join the post-processing before the sums are complete: either ends the build, with the
+    // streams that were forked joined (or waited for, where that fails too).
+    int step_rc = TGPU_OK;
+    auto step = [&](const char *what, hipError_t e) {
+        if (e != hipSuccess && step_rc == TGPU_OK) {
+            c->err = std::string(what) + ": " + hipGetErrorString(e);
+            step_rc = TGPU_E_HIP;
+        }
+        if (e != hipSuccess) (void)hipGetLastError();  // (reported here, not by the next build)
+        return e == hipSuccess;
+    };
     bool used[SideSet::kSide] = {false, false, false};
-    if (fork) (void)hipEventRecord(side->fork, s);
+    if (fork && !step("fork of the side streams", hipEventRecord(side->fork, s))) return step_rc;
     if (prof) std::fill(c->cls_launched.begin(), c->cls_launched.end(), 0);
-    int launch_rc = TGPU_OK;
     for (const int k : order) {
         const int CX = kClassPair[k][0], CY = kClassPair[k][1];
         hipStream_t sk = s;
         if (on[k] > 0) {
             sk = side->s[on[k] - 1];
-            if (!used[on[k] - 1]) (void)hipStreamWaitEvent(sk, side->fork, 0);
+            if (!used[on[k] - 1] && !step("fork of a side stream", hipStreamWaitEvent(sk, side->fork, 0))) break;
             used[on[k] - 1] = true;
         }
         if (prof) (void)hipEventRecord(c->cls_ev[2 * k], s);
@@ -1632,10 +1656,10 @@ static int enqueue_build(tgpu_ctx *c, const BuildBufs &B, const double *P, doubl
                 while (p.split < p.split_max && (waves << (p.split + 1)) <= kSplitWaves) ++p.split;
                 parts[n_part++] = p;
             }
-        launch_rc = kLaunch[k](a, parts, n_part, c->variant[k], mixed, sk);
-        if (launch_rc) {
+        step_rc = kLaunch[k](a, parts, n_part, c->variant[k], mixed, sk);
+        if (step_rc) {
             c->err = "class pair " + std::to_string(k) +
-                     (launch_rc == TGPU_E_STATE ? ": no wavefront-form workspace" : ": too many work-groups");
+                     (step_rc == TGPU_E_STATE ? ": no wavefront-form workspace" : ": too many work-groups");
             break;
         }
         if (prof) {
@@ -1644,11 +1668,11 @@ static int enqueue_build(tgpu_ctx *c, const BuildBufs &B, const double *P, doubl
         }
     }
     for (int q = 0; q < SideSet::kSide; ++q)
-        if (used[q]) {
-            (void)hipEventRecord(side->join[q], side->s[q]);
-            (void)hipStreamWaitEvent(s, side->join[q], 0);
-        }
-    if (launch_rc) return launch_rc;
+        if (used[q] && !(step("join of a side stream", hipEventRecord(side->join[q], side->s[q])) &&
+                         step("join of a side stream", hipStreamWaitEvent(s, side->join[q], 0))) &&
+            s != c->gstream)  // (a capture that fails here is not launched)
+            (void)hipStreamSynchronize(side->s[q]);
+    if (step_rc) return step_rc;
     if (rec_end) (void)hipEventRecord(c->ev1, s);
     if (B.acc_copies > 1)
         acc_reduce_kernel<<<grid_for(c->n_elem), 256, 0, s>>>(B.X, B.Y, (size_t)c->n_elem, B.acc_copies);
@@ -1695,12 +1719,19 @@ extern "C" int tgpu_make_r_JK_device(tgpu_ctx *c, const double *P, double *J, do
         c->g_flags != kflags || c->g_variant != var) {
         drop_graph(c);
         hipGraph_t g = nullptr;
-        const SideLease side(c->device, true);
+        SideLease side(c->device, true);
+        (void)hipGetLastError();  // (not this capture's)
         HIPCHK(c, hipStreamBeginCapture(c->gstream, hipStreamCaptureModeThreadLocal));
-        const int brc = enqueue_build(c, ctx_bufs(c), P, J, K, kflags, c->gstream, side.set, false, false);
-        HIPCHK(c, hipStreamEndCapture(c->gstream, &g));
+        int brc = enqueue_build(c, ctx_bufs(c), P, J, K, kflags, c->gstream, side.set, false, false);
+        const hipError_t le = hipGetLastError(), ee = hipStreamEndCapture(c->gstream, &g);
+        if (!brc && (le != hipSuccess || ee != hipSuccess)) {
+            c->err = std::string("capture of the build: ") + hipGetErrorString(le != hipSuccess ? le : ee);
+            brc = TGPU_E_HIP;
+        }
         if (brc) {
-            (void)hipGraphDestroy(g);
+            // the side streams may still be in the capture: no other build gets them
+            side.discard();
+            if (g) (void)hipGraphDestroy(g);
             return brc;
         }
         hipError_t e = hipGraphInstantiate(&c->gexec, g, nullptr, nullptr, 0);
