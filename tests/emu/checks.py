@@ -201,6 +201,39 @@ def kept_workspace():
     fifth.close()
 
 
+def side_streams_per_stream():
+    """Builds on two streams share no side stream, builds on one stream share theirs; with more
+    streams than sets the longest unused set goes round."""
+    e = Emu()
+    mol = water_cluster(1, "STO-3G", seed=1)
+    streams = [e.L.emu_stream() for _ in range(11)]
+    b = [Build(mol), Build(mol)]
+    J0, K0 = b[0].run()
+
+    def side(k, s):
+        b[k].eng.set_stream(s)
+        e.L.emu_clear()
+        J, K = b[k].run()
+        assert abs(J - J0).max() < 1e-14 and abs(K - K0).max() < 1e-14
+        return frozenset(x[1] for x in e.launches()) - {own(s)}
+
+    def own(s):
+        return ctypes.cast(s, ctypes.POINTER(ctypes.c_int))[0]
+    first = side(0, streams[0])
+    assert len(first) == 3
+    assert not first & side(1, streams[1])
+    assert side(1, streams[0]) == first == side(0, streams[0])
+    e.L.emu_execute(0)
+    J0 = K0 = np.full_like(J0, np.nan)
+    sets = []
+    for s in streams:
+        b[0].eng.set_stream(s)
+        e.L.emu_clear()
+        b[0].run()
+        sets.append(frozenset(x[1] for x in e.launches()) - {own(s)})
+    assert all(len(x) == 3 for x in sets) and len(set(sets)) == 8, sets
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
     print("passed")

@@ -37,3 +37,7 @@ def test_failing_runtime_calls(emulated):
 
 def test_kept_workspace(emulated):
     emulated("kept_workspace")
+
+
+def test_side_streams_per_stream(emulated):
+    emulated("side_streams_per_stream")

@@ -489,15 +489,22 @@ static bool wave_by_default(int lp, int lq, int lr, int ls, bool batch, double q
 // joined before post-processing.  Three side streams: with the build's own, one per hardware
 // queue of the process (4).  Small systems gain most (their launches fill a few CUs each):
 // water/6-31G(d) 2.81 -> 1.58 ms, (H2O)8/6-31G(d) 10.5 -> 4.5, (H2O)7/aug-cc-pVDZ J 17.9 ->
-// 9.0; (H2O)32/cc-pVTZ mixed 858 -> 817 (the tails).  A set costs ~2 ms to make, so the sets of a device are shared by
-// its contexts: a call holds one while it enqueues (no other thread puts work on it
-// meanwhile, nor takes part in its capture) and gives it back when the build is enqueued;
-// later builds on the set queue behind.  At most kMost sets per device (a call that finds
-// none runs its launches in series), one kept when the device's last context goes.
+// 9.0; (H2O)32/cc-pVTZ mixed 858 -> 817 (the tails).  A set costs ~2 ms to make, so the sets
+// of a device are shared by its contexts: a call holds one while it enqueues (no other thread
+// puts work on it meanwhile, nor takes part in its capture) and gives it back when the build
+// is enqueued; later builds on the set queue behind.  Builds on one stream use one set and
+// those on another stream another, so that streams don't queue behind each other here: two
+// threads building (H2O)8/6-31G(d) 4.1 ms a pair with one set for both, 3.8 with two;
+// (H2O)2/6-31G(d) enqueued behind (H2O)24/6-311G(d,p) on another stream 24.4 against 18 ms
+// with 16 hardware queues, 25.8 against 25.0 with the default four, which both share.  At
+// most kMost sets per device (beyond, the longest unused goes round; a call that finds none
+// idle runs its launches in series), kKept kept when the device's last context goes.
 struct SideSet {
     static constexpr int kSide = 3;
     hipStream_t s[kSide] = {nullptr, nullptr, nullptr};
     hipEvent_t fork = nullptr, join[kSide] = {nullptr, nullptr, nullptr};
+    bool used = false;
+    hipStream_t last = nullptr;  // the stream of its last build
 
     bool make()
     {
@@ -518,30 +525,58 @@ struct SideSet {
 };
 
 struct SidePool {
-    static constexpr int kMost = 8;
+    static constexpr int kMost = 8, kKept = 4;
     static std::mutex mu;
-    static std::vector<SideSet *> idle[kMaxDevices];
+    static std::vector<SideSet *> idle[kMaxDevices];  // the longest unused first
     static int made[kMaxDevices], n_ctx[kMaxDevices];
 
-    // an idle set, or (create) a new one on the current device; nullptr if there is none
-    static SideSet *get(int device, bool create)
+    // the idle set whose last build was on stream s, else one without a build yet (-1: none)
+    static int find(int device, hipStream_t s)
     {
-        std::lock_guard<std::mutex> lock(mu);
-        if (!idle[device].empty()) {
-            SideSet *p = idle[device].back();
-            idle[device].pop_back();
-            return p;
+        int fresh = -1;
+        for (int k = 0; k < (int)idle[device].size(); ++k) {
+            const SideSet *p = idle[device][k];
+            if (p->used && p->last == s) return k;
+            if (!p->used) fresh = k;
         }
+        return fresh;
+    }
+    // (create) a new set on the current device into idle; whether there is one
+    static bool add(int device)
+    {
         int now = -1;
-        if (!create || made[device] >= kMost || hipGetDevice(&now) != hipSuccess || now != device) return nullptr;
+        if (made[device] >= kMost || hipGetDevice(&now) != hipSuccess || now != device) return false;
         SideSet *p = new SideSet();
         if (!p->make()) {
             delete p;
             (void)hipGetLastError();  // the build goes on without
-            return nullptr;
+            return false;
         }
         ++made[device];
+        idle[device].push_back(p);
+        return true;
+    }
+    // a set for a build on stream s: one that builds on s used, or an unused or (create) new
+    // one, else the longest unused; nullptr if none is idle
+    static SideSet *get(int device, hipStream_t s, bool create)
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        std::vector<SideSet *> &v = idle[device];
+        int k = find(device, s);
+        if (k < 0 && create && add(device)) k = (int)v.size() - 1;
+        if (k < 0) k = 0;
+        if (v.empty()) return nullptr;
+        SideSet *p = v[k];
+        v.erase(v.begin() + k);
+        p->used = true;
+        p->last = s;
         return p;
+    }
+    // makes a set ready for the first build
+    static void ensure(int device)
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        if (idle[device].empty()) add(device);
     }
     static void put(int device, SideSet *p)
     {
@@ -565,9 +600,9 @@ struct SidePool {
     {
         std::lock_guard<std::mutex> lock(mu);
         if (--n_ctx[device] > 0) return;
-        while (idle[device].size() > 1) {
-            delete idle[device].back();
-            idle[device].pop_back();
+        while ((int)idle[device].size() > kKept) {
+            delete idle[device].front();
+            idle[device].erase(idle[device].begin());
             --made[device];
         }
     }
@@ -580,7 +615,7 @@ int SidePool::made[kMaxDevices], SidePool::n_ctx[kMaxDevices];
 struct SideLease {
     const int device;
     SideSet *set;
-    SideLease(int d, bool create) : device(d), set(SidePool::get(d, create)) {}
+    SideLease(int d, hipStream_t s, bool create) : device(d), set(SidePool::get(d, s, create)) {}
     ~SideLease() { SidePool::put(device, set); }
     void discard()
     {
@@ -1403,7 +1438,7 @@ extern "C" int tgpu_schwarz(tgpu_ctx *c, double *max_I)
             SidePool::add_ctx(c->device);
             c->counted = true;
         }
-        SidePool::put(c->device, SidePool::get(c->device, true));
+        SidePool::ensure(c->device);
         c->have_schwarz = true;
     }
     if (max_I) std::memcpy(max_I, c->maxI_tonto.data(), sizeof(double) * c->n_pairs);
@@ -1704,7 +1739,7 @@ extern "C" int tgpu_make_r_JK_device(tgpu_ctx *c, const double *P, double *J, do
     }
     const int kflags = flags & (TGPU_JK_MIXED | TGPU_J_ONLY | TGPU_K_ONLY);
     if (!(flags & TGPU_JK_GRAPH)) {
-        const SideLease side(c->device, true);
+        const SideLease side(c->device, c->stream, true);
         if (int rc = enqueue_build(c, ctx_bufs(c), P, J, K, kflags, c->stream, side.set, true, true)) return rc;
         c->timed = true;
         HIPCHK(c, hipGetLastError());
@@ -1719,7 +1754,7 @@ extern "C" int tgpu_make_r_JK_device(tgpu_ctx *c, const double *P, double *J, do
         c->g_flags != kflags || c->g_variant != var) {
         drop_graph(c);
         hipGraph_t g = nullptr;
-        SideLease side(c->device, true);
+        SideLease side(c->device, c->stream, true);
         (void)hipGetLastError();  // (not this capture's)
         HIPCHK(c, hipStreamBeginCapture(c->gstream, hipStreamCaptureModeThreadLocal));
         int brc = enqueue_build(c, ctx_bufs(c), P, J, K, kflags, c->gstream, side.set, false, false);
@@ -1830,7 +1865,7 @@ extern "C" int tgpu_make_r_JK_device_noalloc(tgpu_ctx *c, const double *P, doubl
     B.acc_copies = 1;
     B.counter_copies = copies;
     const int kflags = flags & (TGPU_JK_MIXED | TGPU_J_ONLY | TGPU_K_ONLY);
-    const SideLease side(c->device, false);  // (a new set would be an allocation)
+    const SideLease side(c->device, c->stream, false);  // (a new set would be an allocation)
     if (int rc = enqueue_build(c, B, P, J, K, kflags, c->stream, side.set, true, true)) return rc;
     // the context's own counters take this build's, so tgpu_get_stats reports it
     const int n_cnt = TGPU_COUNTER_COPIES * TGPU_COUNTER_STRIDE;
@@ -1876,7 +1911,7 @@ extern "C" int tgpu_make_u_JK_device(tgpu_ctx *c, const double *Pa, const double
     if ((rc = dalloc(c, c->d_uJ, nn)) || (rc = dalloc(c, c->d_uK, nn))) return rc;
     // the timing events bracket all three passes; the class counters are the Pa pass's
     const BuildBufs B = ctx_bufs(c);
-    const SideLease side(c->device, true);
+    const SideLease side(c->device, c->stream, true);
     if ((rc = enqueue_build(c, B, Pb, c->d_uJ.p, c->d_uK.p, flags, c->stream, side.set, true, false, Pa, 1)) ||
         (rc = enqueue_build(c, B, Pb, Jb, Kb, flags, c->stream, side.set, false, false, Pa, 0)) ||
         (rc = enqueue_build(c, B, Pa, Ja, Ka, flags, c->stream, side.set, false, true, Pb, 0)))
