@@ -1,6 +1,7 @@
 """Checks on the library built for the CPU, each run by tests/test_emu.py in a process of its
 own: checks.py NAME (TONTO_GPU_LIB names the library, the address sanitizer is preloaded)."""
 import ctypes
+import dataclasses
 import os
 import sys
 
@@ -8,6 +9,8 @@ sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspa
 
 import numpy as np  # noqa: E402
 
+import oracle.oracle as oracle  # noqa: E402
+from tonto_amd.basis import Molecule  # noqa: E402
 from tonto_amd.geometry import water_cluster  # noqa: E402
 from tonto_amd.gpu import JKEngine, TGPUError, lib  # noqa: E402
 
@@ -232,6 +235,86 @@ def side_streams_per_stream():
         b[0].run()
         sets.append(frozenset(x[1] for x in e.launches()) - {own(s)})
     assert all(len(x) == 3 for x in sets) and len(set(sets)) == 8, sets
+
+
+def _spd_system():
+    """Four atoms far enough apart that quartets over all four lose primitive pairs, some all of
+    them; contracted and single primitives; 12 shells."""
+    m = Molecule.from_angstrom(["O"] * 4, [[0, 0, 0], [2.7, 0.4, -0.3], [0.9, 5.6, 0.5], [6.1, 1.0, 4.2]], "6-31G(d)")
+    shells, bf = [], 0
+    for s in m.shells:
+        n = len(s.exps)
+        if n > (3 if s.atom == 0 else 1) or (s.atom == 0 and n == 1 and s.l < 2):
+            continue
+        shells.append(dataclasses.replace(s, first_bf=bf))
+        bf += s.n_comp
+    m.shells, m.n_bf = shells, bf
+    return m
+
+
+def _compare(eng, mol, P, cut, mixed, tol):
+    J, K = eng.make_r_JK(P, mixed=mixed)
+    Jo, Ko, so = oracle.OracleSystem(mol).make_r_JK(P, schwarz=cut, max_I=eng.schwarz(), return_stats=True)
+    st = eng.stats()
+    print("max|dJ| %.1e max|dK| %.1e, %d quartets" % (abs(J - Jo).max(), abs(K - Ko).max(), st["quartets"]), flush=True)
+    assert st["quartets"] == so["quartets"] and st["prim_quartets"] == so["prim_quartets"]
+    assert max(abs(J - Jo).max(), abs(K - Ko).max()) <= tol
+    return st
+
+
+def wavefront_forms():
+    """Every class pair up to d shells in the wavefront form (FP64, FP32 and both in a build; the
+    last team of a chunk without a quartet, primitive lists that are empty, several passes over
+    rows and columns) and the lane form, against the oracle; the Schwarz table in both bases."""
+    mol = _spd_system()
+    o = oracle.OracleSystem(mol)
+    P = _density(mol.n_bf, 5)
+    for thr, tol in ((1e-9, 1e-11), (1e30, 2e-5), (1e-3, 2e-5)):
+        e = JKEngine(mol, schwarz=1e-13, fp32_threshold=thr)
+        assert abs(e.schwarz() - o.schwarz()).max() < 1e-13
+        for k in range(21):
+            e.set_variant(k, 1)
+            e.set_ket_chunk(k, (16, 32, 64)[k % 3])
+        st = _compare(e, mol, P, 1e-13, thr > 1e-9, tol)
+        assert (st["fp32_quartets"] > 0) == (thr > 1e-9)
+    assert st["fp32_quartets"] < st["quartets"]
+    e = JKEngine(mol, schwarz=1e-13)
+    _compare(e, mol, P, 1e-13, False, 1e-11)
+    e = JKEngine(mol, spherical=True)
+    assert abs(e.schwarz() - o.schwarz_sph()).max() < 1e-13
+
+
+def lane_forms():
+    """The lane form's kinds of K rows (one bra pair per work-group, a wavefront's own; all of
+    them, some, none in LDS), a batch, J or K alone, UHF and the allocation-free build."""
+    mol = _spd_system()
+    P = _density(mol.n_bf, 6)
+    for kets, budget in (("0", None), ("0", "15900"), ("1000000", None), ("1000000", "24000"), ("1000000", "15000")):
+        os.environ["TGPU_KROW_MIN_KETS"] = kets
+        if budget:
+            os.environ["TGPU_KROW_BUDGET"] = budget
+        e = JKEngine(mol, schwarz=1e-13)
+        os.environ.pop("TGPU_KROW_BUDGET", None)
+        _compare(e, mol, P, 1e-13, False, 1e-11)
+    del os.environ["TGPU_KROW_MIN_KETS"]
+    max_I = e.schwarz()
+    o = oracle.OracleSystem(mol)
+    Jo, Ko = o.make_r_JK(P, schwarz=1e-13, max_I=max_I)
+    J, K = np.zeros_like(P), np.zeros_like(P)
+    for only in ("J", "K", None):
+        e.make_r_JK_device_noalloc(P.ctypes.data, J.ctypes.data, K.ctypes.data, only=only)
+        assert only == "K" or abs(J - Jo).max() < 1e-11
+        assert only == "J" or abs(K - Ko).max() < 1e-11
+    P2 = _density(mol.n_bf, 7)
+    for x, y in zip(e.make_u_JK(P, P2), o.make_u_JK(P, P2, schwarz=1e-13, max_I=max_I)):
+        assert abs(x - y).max() < 1e-11
+    mols = [water_cluster(1, "STO-3G", seed=1), mol, water_cluster(2, "STO-3G", seed=2)]
+    Ps = [_density(m.n_bf, i) for i, m in enumerate(mols)]
+    b = JKEngine(mols, schwarz=1e-12)
+    max_I = b.schwarz()
+    for i, (m, p, J, K) in enumerate(zip(mols, Ps, *b.make_r_JK(Ps))):
+        Jo, Ko = oracle.OracleSystem(m).make_r_JK(p, schwarz=1e-12, max_I=max_I[b.pair_off[i]:b.pair_off[i + 1]])
+        assert max(abs(J - Jo).max(), abs(K - Ko).max()) < 1e-11
 
 
 if __name__ == "__main__":

@@ -1,15 +1,23 @@
 // Lanes as fibers, and the log of the runtime's calls.
 #include "hip/hip_runtime.h"
 #include <string>
-#include <ucontext.h>
 #include <vector>
+
+// Saves the callee-saved registers and the stack pointer in *save and goes on at `to` (x86-64).
+// swapcontext would do, but its system call per switch is most of a run's time.
+extern "C" __attribute__((naked, noinline)) void emu_switch(void **save, void *to)
+{
+    asm("push %rbx; push %rbp; push %r12; push %r13; push %r14; push %r15;"
+        "mov %rsp, (%rdi); mov %rsi, %rsp;"
+        "pop %r15; pop %r14; pop %r13; pop %r12; pop %rbp; pop %rbx; ret");
+}
 
 namespace emu {
 dim3 tIdx, bIdx, bDim, gDim;
 unsigned char *dyn_lds;
 namespace {
 struct Fiber {
-    ucontext_t ctx;
+    void *sp;
     bool done;
     char *stack;
     long turn[64];          // exchanges done per distance
@@ -17,7 +25,7 @@ struct Fiber {
 };
 constexpr size_t kStack = 1 << 20;
 std::vector<Fiber *> fibers;
-ucontext_t scheduler;
+void *scheduler;
 int cur, n_lanes;
 const std::function<void()> *body_fn;
 long wave_gen[16], wave_cnt[16], block_gen, block_cnt;
@@ -28,12 +36,12 @@ void body()
 {
     (*body_fn)();
     fibers[cur]->done = true;
-    swapcontext(&fibers[cur]->ctx, &scheduler);
+    emu_switch(&fibers[cur]->sp, scheduler);
 }
 void yield()
 {
     const int me = cur;
-    swapcontext(&fibers[me]->ctx, &scheduler);
+    emu_switch(&fibers[me]->sp, scheduler);
 }
 int alive(int a, int b)
 {
@@ -147,11 +155,10 @@ void launch(const char *name, dim3 g, dim3 b, size_t lds, hipStream_t s, const s
                 Fiber *f = fibers[i];
                 f->done = false;
                 memset(f->turn, 0, sizeof f->turn);
-                getcontext(&f->ctx);
-                f->ctx.uc_stack.ss_sp = f->stack;
-                f->ctx.uc_stack.ss_size = kStack;
-                f->ctx.uc_link = &scheduler;
-                makecontext(&f->ctx, body, 0);
+                // the switch pops six registers and returns into body(), which never returns
+                void **top = reinterpret_cast<void **>(f->stack + kStack) - 1;  // 8 mod 16, as after a call
+                top[-1] = reinterpret_cast<void *>(&body);
+                f->sp = top - 7;
             }
             memset(wave_cnt, 0, sizeof wave_cnt);
             block_cnt = 0;
@@ -162,7 +169,7 @@ void launch(const char *name, dim3 g, dim3 b, size_t lds, hipStream_t s, const s
                     cur = i;
                     tIdx = dim3(i, 0, 0);
                     bIdx = dim3(bx, by, 0);
-                    swapcontext(&scheduler, &fibers[i]->ctx);
+                    emu_switch(&scheduler, fibers[i]->sp);
                     left += !fibers[i]->done;
                 }
             }

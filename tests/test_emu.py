@@ -41,3 +41,11 @@ def test_kept_workspace(emulated):
 
 def test_side_streams_per_stream(emulated):
     emulated("side_streams_per_stream")
+
+
+def test_wavefront_forms(emulated):
+    emulated("wavefront_forms")
+
+
+def test_lane_forms(emulated):
+    emulated("lane_forms")
