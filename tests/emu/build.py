@@ -1,5 +1,5 @@
 """Builds the library's HIP sources for the CPU (hip/hip_runtime.h, emu.cpp) with the address
-sanitizer; the class pairs with f shells are stubs that only log."""
+sanitizer."""
 import os
 import re
 import shutil
@@ -60,24 +60,12 @@ def build(out):
     for f in ("tgpu_device.h", "tgpu_host.hip", "jk_class.hip"):
         text = convert(open(os.path.join(src, f)).read())
         open(os.path.join(src, f), "w").write(text)
-    stubs = ['#include "tgpu_device.h"']
-    jobs = [(os.path.join(src, "tgpu_host.hip"), "host", []), (os.path.join(HERE, "emu.cpp"), "emu", [])]
+    jobs = [(os.path.join(src, "tgpu_host.hip"), "host", []), (os.path.join(HERE, "emu.cpp"), "emu", []),
+            (shutil.copy(os.path.join(HERE, "shapes.cpp"), src), "shapes", [])]
     for lp, lq, lr, ls, heavy in class_list():
-        name = f"{lp}{lq}{lr}{ls}"
-        if lp <= 2:
-            jobs.append((os.path.join(src, "jk_class.hip"), "jk_" + name,
-                         [f"-DTGPU_LP={lp}", f"-DTGPU_LQ={lq}", f"-DTGPU_LR={lr}", f"-DTGPU_LS={ls}",
-                          f"-DTGPU_HEAVY={heavy}"]))
-            continue
-        stubs.append(f"int tgpu_launch_jk_{name}(const JKArgs &, const JKPart *, int, int, bool, hipStream_t s)"
-                     f' {{ emu::launch("stub_{name}", 1, 1, 0, s, [] {{}}); return TGPU_OK; }}')
-        stubs.append(f"size_t tgpu_wave_ws_{name}() {{ return {1000 if name == '3333' else 0}; }}")
-        if (lp, lq) == (lr, ls):
-            stubs.append(f"void tgpu_launch_schwarz_{lp}{lq}(const DevPairs &, const DevPrims &, int start, int n, double"
-                         " *maxI, double *, long long, int, hipStream_t) { for (int i = 0; i < n; ++i) maxI[start + i] = 1.0; }")
-    open(os.path.join(src, "stubs.cpp"), "w").write("\n".join(stubs) + "\n")
-    jobs.append((os.path.join(src, "stubs.cpp"), "stubs", []))
-    jobs.append((shutil.copy(os.path.join(HERE, "shapes.cpp"), src), "shapes", []))
+        jobs.append((os.path.join(src, "jk_class.hip"), f"jk_{lp}{lq}{lr}{ls}",
+                     [f"-DTGPU_LP={lp}", f"-DTGPU_LQ={lq}", f"-DTGPU_LR={lr}", f"-DTGPU_LS={ls}",
+                      f"-DTGPU_HEAVY={heavy}"]))
 
     def compile_one(job):
         obj = os.path.join(out, job[1] + ".o")

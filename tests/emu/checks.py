@@ -252,6 +252,20 @@ def _spd_system():
     return m
 
 
+def _f_system():
+    """Three atoms with an f, a d, a p and an s shell (cc-pVTZ), the first s contracted."""
+    m = Molecule.from_angstrom(["O"] * 4, [[0, 0, 0], [2.7, 0.4, -0.3], [0.9, 5.6, 0.5], [6.1, 1.0, 4.2]], "cc-pVTZ")
+    shells, bf, seen = [], 0, set()
+    for s in m.shells:
+        if (s.atom, s.l) in seen or (s.l < 2 and len(s.exps) > 1 and (s.atom or s.l)) or (s.atom == 3 and s.l > 1):
+            continue
+        seen.add((s.atom, s.l))
+        shells.append(dataclasses.replace(s, first_bf=bf))
+        bf += s.n_comp
+    m.shells, m.n_bf = shells, bf
+    return m
+
+
 def _compare(eng, mol, P, cut, mixed, tol):
     J, K = eng.make_r_JK(P, mixed=mixed)
     Jo, Ko, so = oracle.OracleSystem(mol).make_r_JK(P, schwarz=cut, max_I=eng.schwarz(), return_stats=True)
@@ -280,6 +294,30 @@ def wavefront_forms():
     assert st["fp32_quartets"] < st["quartets"]
     e = JKEngine(mol, schwarz=1e-13)
     _compare(e, mol, P, 1e-13, False, 1e-11)
+    e = JKEngine(mol, spherical=True)
+    assert abs(e.schwarz() - o.schwarz_sph()).max() < 1e-13
+
+
+def f_shells():
+    """Class pairs with f shells: both forms, the workspace as large as its launches need and as
+    small as the allocation-free build may leave it, both bases."""
+    mol = _f_system()
+    o = oracle.OracleSystem(mol)
+    P = _density(mol.n_bf, 5)
+    for wave, thr, tol in ((1, 1e-9, 1e-11), (1, 1e-3, 2e-5), (0, 1e-9, 1e-11)):
+        e = JKEngine(mol, schwarz=1e-12, fp32_threshold=thr)
+        assert abs(e.schwarz() - o.schwarz()).max() < 1e-13
+        for k in range(55):
+            try:
+                e.set_variant(k, wave)
+            except TGPUError:  # only the wavefront form
+                pass
+            e.set_ket_chunk(k, (16, 32, 64)[k % 3])
+        _compare(e, mol, P, 1e-12, thr > 1e-9, tol)
+    Jo, Ko = o.make_r_JK(P, schwarz=1e-12, max_I=e.schwarz())
+    J, K = np.zeros_like(P), np.zeros_like(P)
+    e.make_r_JK_device_noalloc(P.ctypes.data, J.ctypes.data, K.ctypes.data)
+    assert max(abs(J - Jo).max(), abs(K - Ko).max()) < 1e-11
     e = JKEngine(mol, spherical=True)
     assert abs(e.schwarz() - o.schwarz_sph()).max() < 1e-13
 

@@ -49,3 +49,7 @@ def test_wavefront_forms(emulated):
 
 def test_lane_forms(emulated):
     emulated("lane_forms")
+
+
+def test_f_shells(emulated):
+    emulated("f_shells")
