@@ -267,8 +267,8 @@ def main():
     a = ap.parse_args()
     if a.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
         print("bench.py measures one GPU: this build has no multi-GPU path "
-              "(the J/K build would shard by bra shell pairs with one all-reduce of J and K; "
-              "see DESIGN.md).  Run with --gpus 1.", file=sys.stderr)
+              "(the J/K build would shard by bra shell pairs with one all-reduce of J and K).  "
+              "Run with --gpus 1.", file=sys.stderr)
         sys.exit(2)
 
     import torch
@@ -351,13 +351,14 @@ def main():
     steps64 = min(a.steps, 3)
     wall64 = time_steps(eng, lambda: scf.jk(P, "full"), steps64, 1, torch.cuda.synchronize)
     st64 = eng.stats()
+    t64 = class_ms(eng, lambda: scf.jk(P, "full"), 1)
     q = stmx["quartets"]
     value = q * a.steps / wallmx
     fmx, pmx = build_flops(cntmx)
     for kk, cp in enumerate(class_pairs()):
         if cntmx[kk][0]:
-            log("class (%d%d|%d%d) quartets %11d prim %12d fp32 %11d | mixed %9.3f ms %6.2f TF"
-                % (*cp, cntmx[kk][0], cntmx[kk][1], cntmx[kk][2], tmx[kk], pmx[kk] / max(tmx[kk], 1e-9) / 1e9))
+            log("class (%d%d|%d%d) quartets %11d prim %12d fp32 %11d | mixed %9.3f ms %6.2f TF, FP64 %9.3f ms"
+                % (*cp, cntmx[kk][0], cntmx[kk][1], cntmx[kk][2], tmx[kk], pmx[kk] / max(tmx[kk], 1e-9) / 1e9, t64[kk]))
     ms_step = wallmx / a.steps * 1e3
     log(f"mixed build {ms_step:.1f} ms ({fmx / (ms_step * 1e-3) / 1e12:.2f} TF algorithmic), "
         f"FP64 build {wall64 / steps64 * 1e3:.1f} ms")

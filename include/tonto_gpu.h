@@ -4,8 +4,7 @@
  *   MOLECULE.FOCK:make_r_JK_engine(J,K,P)   (foofiles/molecule.fock.foo:1365-1505),
  * which Tonto calls from make_r_Fock_mx (molecule.fock.foo:125) inside every SCF
  * iteration (molecule.scf.foo:1562-1620).  A Fortran caller binds these functions with
- * iso_c_binding; the shim that replaces the body of make_r_JK_engine is shown in
- * INTEGRATION.md.
+ * iso_c_binding; a shim in place of the body of make_r_JK_engine calls them.
  *
  * Conventions
  *  - Every function returns 0 on success and a non-zero TGPU_E_* code on failure;

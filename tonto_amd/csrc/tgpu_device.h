@@ -364,12 +364,12 @@ struct JKArgs {
     // KROWS form, single molecules: n_shell shells; pmrow (set per launch) 1 when the bra
     // pair's two P_max rows (2 n_shell doubles) are staged in LDS after the density rows
     int n_shell, pmrow;
-    // KROWS form, single molecules: the K columns a class pair touches are the functions
+    // K rows in LDS: the K columns a class pair touches are the functions
     // of its ket shells' two angular momenta, so an LDS row holds only those, numbered
     // within each momentum.  kcol[pair] = pack16(number of the pair's first function
     // among the functions of its first shell's momentum, the same for its second shell);
-    // the functions of momentum l are kcol_map[kcol_lofs[l] .. kcol_lofs[l + 1]).  Null
-    // for batches.
+    // the functions of momentum l are kcol_map[kcol_lofs[l] .. kcol_lofs[l + 1]) (a single
+    // molecule's; all 0 for batches, which have no KROWS form).
     const int *kcol;
     const int *kcol_map;
     int kcol_lofs[TGPU_LMAX + 2];
@@ -1033,8 +1033,8 @@ namespace rows_form {
 //   columns  lane c = (r, s) reads column c of (e0|rs), transfers the bra in registers and
 //            digests its NPQ integrals there: ket-side J by one atomic, K as partial sums
 //            over q or p, through LDS, added over s or r by one lane per K element.
-// LDS holds NE NRS values a quartet instead of two buffers of up to 1.5 NPQ NRS, so that 2 to
-// 3 wavefronts fit a SIMD.  The classes with f shells keep the level form below: their rows
+// LDS holds NE NRS values a quartet instead of two buffers of up to 1.5 NPQ NRS; the registers
+// (up to 256) then leave 2 wavefronts per SIMD (1.7 to 2.2 measured at (H2O)64/cc-pVTZ).  The classes with f shells keep the level form below: their rows
 // and columns (25 to 100 values a lane) do not fit the registers.
 // ----------------------------------------------------------------------------------
 template <int L1, int L2> struct PairForm;

@@ -465,17 +465,17 @@ static const bool kHeavy[NQCLS] = {
 };
 
 // Default kernel form per class pair: the lane-per-quartet form for every class pair that
-// has one, with these exceptions (class times of one build, lane against wavefront form):
-//   (ff|ss)               0.93 against 0.67 ms at (H2O)12/cc-pVTZ, 4.4 against 4.3 at (H2O)32
+// has one, with these exceptions (class times of one FP64 build, lane against wavefront form):
+//   (ff|ss)               0.77 against 0.64 ms at (H2O)12/cc-pVTZ, 3.1 against 2.6 at (H2O)32
 //                         (its lane kernel updates K globally);
-//   (dp|pp) in batches    13.0 against 12.6 ms for 256 clusters in 6-31G(d,p), where
-//                         (ps|ps)-like classes are at 40 against 136 and (dd|ps) at 3.8
-//                         against 10.4;
+//   (dp|pp) in batches    13.4 against 12.4 ms for 256 clusters in 6-31G(d,p), where (dp|ds)
+//                         is at 7.8 against 12.0 and (dd|ps) at 3.7 against 10.4;
 //   more than 100 integrals and few quartets (fewer than 2^19 bra-ket pairs of a single
 //   molecule): the lane kernels of these hold 400 to 512 registers, one wavefront per SIMD,
-//   and a small system does not fill the lanes: (dd|ps) 0.47 against 0.14 ms at
-//   (H2O)8/6-31G(d), (fp|ds) 1.02 against 0.48 at (H2O)5/cc-pVTZ, but (fp|ds) 1.3 against
-//   2.8 at (H2O)12/cc-pVTZ.
+//   and a small system does not fill the lanes: (dd|ps) 0.33 against 0.09 ms at
+//   (H2O)8/6-31G(d), (fp|ds) 1.26 against 0.36 at (H2O)5/cc-pVTZ, but (fp|ds) 1.06 against
+//   1.62 at (H2O)12/cc-pVTZ.  Near the line both ways occur: at (H2O)8/cc-pVTZ, above it,
+//   (fp|ds) 0.86 against 1.11, (fd|ps) 1.27 against 0.83.
 // tgpu_autotune re-decides per context.
 static bool wave_by_default(int lp, int lq, int lr, int ls, bool batch, double quartets)
 {

@@ -1,6 +1,6 @@
 ! iso_c_binding interface to libtonto_gpu (include/tonto_gpu.h) for Tonto's Fortran.
 ! A Tonto build links libtonto_gpu.so and calls these from MOLECULE.FOCK:make_r_JK_engine
-! (foofiles/molecule.fock.foo:1365-1505); see INTEGRATION.md for the shim.
+! (foofiles/molecule.fock.foo:1365-1505).
 module tonto_gpu_mod
    use, intrinsic :: iso_c_binding
    implicit none
