@@ -112,15 +112,13 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, cons
         for (int k0 = 0, k1; k0 < n_part; k0 = k1) {
             k1 = launch_end(groups, n_part, k0, kMostThreads / 256);
             int rows_grid = 0, glob_grid = 0;
-            rows.n_part = glob.n_part = 0;
+            rows.clear();
+            glob.clear();
             for (int k = k0; k < k1; ++k) {
                 const bool r = in_rows(parts[k]);
-                JKLaunch &L = r ? rows : glob;
-                JKPart &p = L.part[L.n_part++];
-                p = parts[k];
-                p.gx = p.gy = 1;
                 int &grid = r ? rows_grid : glob_grid;
-                p.first = grid;
+                JKPart &p = (r ? rows : glob).add(parts[k], grid);
+                p.gx = p.gy = 1;
                 grid += (int)groups[k];
             }
 #if !(TGPU_LP == 3 && TGPU_LQ == 3 && TGPU_LR == 0 && TGPU_LS == 0)
@@ -186,14 +184,12 @@ int TGPU_LAUNCH_NAME_X(TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS)(const JKArgs &a, cons
     for (int k0 = 0, k1; k0 < n_part; k0 = k1) {
         k1 = launch_end(groups, n_part, k0, kMostThreads / 64);
         int grid = 0;
-        L.n_part = k1 - k0;
+        L.clear();
         for (int k = k0; k < k1; ++k) {
-            JKPart &p = L.part[k - k0];
-            p = parts[k];
+            JKPart &p = L.add(parts[k], grid);
             p.ket_chunk = chunk(p);
             p.gx = (int)plan[k].gx;
             p.gy = (int)plan[k].gy;
-            p.first = grid;
             grid += (int)groups[k];
         }
         jk_wave_kernel<TGPU_LP, TGPU_LQ, TGPU_LR, TGPU_LS, double><<<grid, 64, 0, s>>>(L);
