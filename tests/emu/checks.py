@@ -237,6 +237,22 @@ def side_streams_per_stream():
     assert all(len(x) == 3 for x in sets) and len(set(sets)) == 8, sets
 
 
+def captured_by_the_caller():
+    """A build on a stream that the caller captures makes no stream or event and forks nothing."""
+    e = Emu()
+    b = Build(water_cluster(1, "STO-3G", seed=1))
+    J0, K0 = b.run()
+    s = e.L.emu_stream()
+    ctypes.cast(s, ctypes.POINTER(ctypes.c_int))[1] = 1  # (its capture flag)
+    b.eng.set_stream(s)
+    e.L.emu_clear()
+    J, K = b.run()
+    assert abs(J - J0).max() < 1e-14 and abs(K - K0).max() < 1e-14
+    log = e.log()
+    assert not [x for x in log if "Create" in x[0] or x[0] in ("hipMalloc", "hipStreamWaitEvent")], log
+    assert len({x[1] for x in e.launches()}) == 1
+
+
 def _spd_system():
     """Four atoms far enough apart that quartets over all four lose primitive pairs, some all of
     them; contracted and single primitives; 12 shells."""

@@ -53,3 +53,7 @@ def test_lane_forms(emulated):
 
 def test_f_shells(emulated):
     emulated("f_shells")
+
+
+def test_captured_by_the_caller(emulated):
+    emulated("captured_by_the_caller")

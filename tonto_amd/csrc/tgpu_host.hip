@@ -560,6 +560,9 @@ struct SidePool {
     // one, else the longest unused; nullptr if none is idle
     static SideSet *get(int device, hipStream_t s, bool create)
     {
+        // (nothing is made while the caller captures s; such a build runs in series)
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (s && create && (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone)) create = false;
         std::lock_guard<std::mutex> lock(mu);
         std::vector<SideSet *> &v = idle[device];
         int k = find(device, s);
